@@ -19,8 +19,10 @@
 // accumulator input is a bias that makes the convert and the first multiply
 // one fma (see kDotBiasBits): three instructions per output and block.  A 256-thread workgroup owns a
 // 64 x 64 output tile (four waves of 32 x 32), and the dots of the next block
-// are computed before the current block's are scaled.  Two operand layouts,
-// two ways of feeding the matrix core:
+// are computed before the current block's are scaled.  (Split planes run 16-
+// or 32-row tiles of the 16 x 16 x 32 instruction instead, except large grids
+// over short rows: q4_0_tiled16_kernel.)  Two operand layouts, two ways of
+// feeding the matrix core:
 //   * split planes (the reference's GGML_Q4_0_Q8_0_TILED_LINEAR_KERNEL
 //     contract, ggml_q4_0.py:844-967): activation int8 [M, K] + fp16 scales
 //     [M, B] (2-byte halves or 4-byte words), weight uint32 [B * 8, N] of
@@ -30,6 +32,8 @@
 //   * native 34-byte Q8_0 / 18-byte Q4_0 blocks (the linear's own layout):
 //     the workgroup stages 8 blocks of its rows and columns at a time in LDS,
 //     realigned and with the weight nibbles already converted to int8.
+#include <type_traits>
+
 #include "qxt_common.h"
 
 namespace qxt {
@@ -138,39 +142,40 @@ __device__ __forceinline__ bool half_bits_finite(uint32_t bits16) { return (bits
 // Row of output r (0..15) of a lane: the 32 x 32 MFMA's output layout.
 __device__ __forceinline__ int out_row(int mbase, int r) { return mbase + 8 * (r >> 2) + (r & 3); }
 
-// The exact per-block form, c_b = fl32(fl32(float(dot) * dw) * da) summed in
-// block order, for one lane's 16 outputs (rows out_row(mbase, r), column bn),
-// straight from the split planes in global memory (v_dot4 per 4 k), one
-// output at a time so that it needs few registers.  Only for workgroups
-// whose weight scales are not all finite.
-__device__ __forceinline__ void exact_terms_split(const TiledArgs &t, int mbase, int bn, float (&acc)[16]) {
+// The exact per-block form of one output, c_b = fl32(fl32(float(dot) * dw) *
+// da) summed in block order, straight from the split planes in global memory
+// (v_dot4 per 4 k).  Only for workgroups whose weight scales are not all
+// finite.
+__device__ __forceinline__ float exact_output_split(const TiledArgs &t, int m, int bn) {
     const __amdgpu_buffer_rsrc_t ra = rsrc(t.aq, t.a_extent);
     const __amdgpu_buffer_rsrc_t rw = rsrc(t.wq, t.w_extent);
     const __amdgpu_buffer_rsrc_t ras = rsrc(t.as, t.as_extent);
     const __amdgpu_buffer_rsrc_t rws = rsrc(t.ws, t.ws_extent);
-    const bool n_ok = bn < t.n;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int m = out_row(mbase, r);
-        const bool m_ok = m < t.m;
-        float sum = 0.0f;
+    const bool n_ok = bn < t.n, m_ok = m < t.m;
+    float sum = 0.0f;
 #pragma unroll 1
-        for (int b = 0; b < t.blocks; ++b) {
-            const uint32_t ao = m_ok ? static_cast<uint32_t>(m) * t.aq_stride + b * 32 : kOutOfRange;
-            const uint32_t wo = n_ok ? static_cast<uint32_t>(b * 8) * t.wq_stride + bn * 4 : kOutOfRange;
-            int dot = 0;
+    for (int b = 0; b < t.blocks; ++b) {
+        const uint32_t ao = m_ok ? static_cast<uint32_t>(m) * t.aq_stride + b * 32 : kOutOfRange;
+        const uint32_t wo = n_ok ? static_cast<uint32_t>(b * 8) * t.wq_stride + bn * 4 : kOutOfRange;
+        int dot = 0;
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
-                dot = dot4(static_cast<int>(__builtin_amdgcn_raw_buffer_load_b32(ra, ao + 4 * j, 0, 0)),
-                           static_cast<int>(__builtin_amdgcn_raw_buffer_load_b32(rw, wo + j * t.wq_stride, 0, 0)), dot);
-            const float dw = half_bits_to_float(__builtin_amdgcn_raw_buffer_load_b16(
-                rws, n_ok ? static_cast<uint32_t>(b) * t.ws_stride + bn * 2 : kOutOfRange, 0, 0));
-            const float da = half_bits_to_float(__builtin_amdgcn_raw_buffer_load_b16(
-                ras, m_ok ? static_cast<uint32_t>(m) * t.as_stride + b * t.as_bytes : kOutOfRange, 0, 0));
-            sum = sum + (static_cast<float>(dot) * dw) * da;
-        }
-        acc[r] = sum;
+        for (int j = 0; j < 8; ++j)
+            dot = dot4(static_cast<int>(__builtin_amdgcn_raw_buffer_load_b32(ra, ao + 4 * j, 0, 0)),
+                       static_cast<int>(__builtin_amdgcn_raw_buffer_load_b32(rw, wo + j * t.wq_stride, 0, 0)), dot);
+        const float dw = half_bits_to_float(__builtin_amdgcn_raw_buffer_load_b16(
+            rws, n_ok ? static_cast<uint32_t>(b) * t.ws_stride + bn * 2 : kOutOfRange, 0, 0));
+        const float da = half_bits_to_float(__builtin_amdgcn_raw_buffer_load_b16(
+            ras, m_ok ? static_cast<uint32_t>(m) * t.as_stride + b * t.as_bytes : kOutOfRange, 0, 0));
+        sum = sum + (static_cast<float>(dot) * dw) * da;
     }
+    return sum;
+}
+
+// One lane's 16 outputs (rows out_row(mbase, r), column bn) that way, one at
+// a time so that it needs few registers.
+__device__ __forceinline__ void exact_terms_split(const TiledArgs &t, int mbase, int bn, float (&acc)[16]) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = exact_output_split(t, out_row(mbase, r), bn);
 }
 
 // The same from native 34-byte Q8_0 / 18-byte Q4_0 blocks (2-byte aligned:
@@ -369,6 +374,236 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, COL
             if (m < t.m)
                 reinterpret_cast<float *>(reinterpret_cast<uint8_t *>(t.y) + static_cast<size_t>(m) * t.y_stride)[t.ocol0 + bn] =
                     COLUMN ? acc[4 * q + e] * cs : acc[4 * q + e];
+        }
+}
+
+// ------------------------------------- split planes, 16 x 16 tiles per wave
+//
+// The same arithmetic (biased dots) with one v_mfma_i32_16x16x32_i8 per block
+// and 16 x 16 output tile.  A workgroup of four waves owns 16 RT rows x 64
+// columns; RT = 1 gives a short prompt four times the waves of the 64 x 64
+// tiles (M = 77, N = 2048 ran 64 workgroups, one wave of 16 outputs per lane
+// and block on each SIMD they reached: 37.5 us, a serial chain of K / 32
+// blocks), RT = 2 halves the weight words read per output for larger grids.
+// What bounds it then: RT = 1, the chain of K / 32 blocks per wave (72 ns a
+// block with one wave per SIMD); RT = 2, VALU and L2 reads of the weight words
+// together.  What took the chain from 100 to 72 ns a block, measured at M = 16,
+// K = 5632: every LDS read a group of blocks ahead of its use; activation
+// fragments in lane order (the row-major order conflicted two ways); the four
+// activation scales of a lane broadcast by DPP from one register per four
+// blocks (a 16-byte LDS read per block kept the LDS busy 77 of 81 thousand
+// cycles at M = 512).  Thirty-two blocks of weight words in flight instead of
+// sixteen spill (18.3 against 15.5 us).
+// Measured on MI355X against the 64 x 64 tiles, bit-identical (K x N, rows):
+// 5632 x 2048: 77 rows 37.5 -> 16.2 us, 256 37.8 -> 21.3, 512 38.4 -> 32.2;
+// 2048 x 5632: 77 rows 16.5 -> 10.5, 256 26.3 -> 22.3, 1024 72.6 -> 68.1;
+// 4096 x 11008: 160 rows 66.0 -> 48.0, 512 149 -> 133 us.
+template <int RT>
+struct Split16 {
+    static constexpr int kRows = 16 * RT;
+    static constexpr int kBlocks = RT == 1 ? 32 : 16;     // blocks staged per round
+    static constexpr int kPitch = kRows * 32 + 8;         // bytes of one staged block's activation rows
+    static constexpr int kSub = 4;                        // blocks multiplied, then scaled, together
+    static constexpr int kAhead = 16;                     // blocks of weight words in flight
+    static constexpr int kPieces = kBlocks * kRows * 2 / kThreads;   // 16-byte activation pieces per thread
+    static constexpr int kDa = kBlocks * kRows / kThreads;           // activation scales per thread
+    static constexpr int kDw = kBlocks * kTile / kThreads;           // weight scales per thread
+    struct Buf {
+        uint8_t a[kBlocks * kPitch];   // 8-byte pieces in lane order: [block][k / 8][row]
+        float da[kBlocks / kSub][64 * RT];  // lane (row / 4, 4 (block % 4) + row % 4)
+        float2 dw[kBlocks][kTile];  // (scale, -kDotBias * scale)
+    };
+};
+
+template <int RT>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 2))) void q4_0_tiled16_kernel(
+    TiledArgs t) {
+    using G = Split16<RT>;
+    __shared__ __attribute__((aligned(16))) typename G::Buf s_buf[2];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int kg = lane >> 4, l16 = lane & 15;
+    const int m0 = blockIdx.y * G::kRows, n0 = blockIdx.x * kTile;
+    const int bn = n0 + wave * 16 + l16;  // column of this lane's weight words and outputs
+    const bool b_ok = bn < t.n;
+
+    const __amdgpu_buffer_rsrc_t ra = rsrc(t.aq, t.a_extent);
+    const __amdgpu_buffer_rsrc_t rw = rsrc(t.wq, t.w_extent);
+    const __amdgpu_buffer_rsrc_t ras = rsrc(t.as, t.as_extent);
+    const __amdgpu_buffer_rsrc_t rws = rsrc(t.ws, t.ws_extent);
+
+    // The next round's activation rows and both scales, in registers until
+    // the round before it is done (zeros past M, N and K).
+    v4u a_raw[G::kPieces];
+    uint32_t da_bits[G::kDa], dw_bits[G::kDw];
+    bool finite = true;
+    auto load_round = [&](int c0) {
+#pragma unroll
+        for (int u = 0; u < G::kPieces; ++u) {
+            const int i = threadIdx.x + u * kThreads;
+            const int r = i / (2 * G::kBlocks), p = i % (2 * G::kBlocks);
+            const bool ok = m0 + r < t.m && c0 + (p >> 1) < t.blocks;
+            a_raw[u] = __builtin_amdgcn_raw_buffer_load_b128(
+                ra, ok ? static_cast<uint32_t>(m0 + r) * t.aq_stride + c0 * 32 + p * 16 : kOutOfRange, 0, 0);
+        }
+#pragma unroll
+        for (int u = 0; u < G::kDa; ++u) {
+            const int i = threadIdx.x + u * kThreads;
+            const int r = i / G::kBlocks, b = c0 + i % G::kBlocks;
+            const bool ok = m0 + r < t.m && b < t.blocks;
+            da_bits[u] = __builtin_amdgcn_raw_buffer_load_b16(
+                ras, ok ? static_cast<uint32_t>(m0 + r) * t.as_stride + b * t.as_bytes : kOutOfRange, 0, 0);
+        }
+#pragma unroll
+        for (int u = 0; u < G::kDw; ++u) {
+            const int i = threadIdx.x + u * kThreads;
+            const int n = n0 + i % kTile, b = c0 + i / kTile;
+            const bool ok = n < t.n && b < t.blocks;
+            dw_bits[u] = __builtin_amdgcn_raw_buffer_load_b16(
+                rws, ok ? static_cast<uint32_t>(b) * t.ws_stride + n * 2 : kOutOfRange, 0, 0);
+        }
+    };
+    auto store_round = [&](typename G::Buf &s) {
+#pragma unroll
+        for (int u = 0; u < G::kPieces; ++u) {
+            const int i = threadIdx.x + u * kThreads;
+            const int r = i / (2 * G::kBlocks), p = i % (2 * G::kBlocks);
+            uint8_t *dst = s.a + (p >> 1) * G::kPitch + (r >> 4) * 512 + (p & 1) * 256 + (r & 15) * 8;
+            *reinterpret_cast<uint2 *>(dst) = make_uint2(a_raw[u][0], a_raw[u][1]);
+            *reinterpret_cast<uint2 *>(dst + 128) = make_uint2(a_raw[u][2], a_raw[u][3]);
+        }
+#pragma unroll
+        for (int u = 0; u < G::kDa; ++u) {
+            const int i = threadIdx.x + u * kThreads;
+            const int r = i / G::kBlocks, b = i % G::kBlocks;
+            s.da[b / G::kSub][(r >> 2) * 16 + (b % G::kSub) * 4 + (r & 3)] = half_bits_to_float(da_bits[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < G::kDw; ++u) {
+            const int i = threadIdx.x + u * kThreads;
+            const float d = half_bits_to_float(dw_bits[u]);
+            s.dw[i / kTile][i % kTile] = make_float2(d, d * -kDotBias);
+            finite = finite && half_bits_finite(dw_bits[u]);
+        }
+    };
+    load_round(0);
+
+    // Lane (kg, l16) holds k = 8 kg .. 8 kg + 7 of its row or column: two
+    // consecutive weight word rows, 8 consecutive activation bytes.
+    // Rows past K are past the descriptor's range and read zeros (the offset
+    // does not wrap: split16_supported).
+    uint32_t woff = b_ok ? static_cast<uint32_t>(2 * kg) * t.wq_stride + bn * 4 : t.w_extent;
+    const uint32_t wstep = 8u * t.wq_stride;
+    uint32_t ring[G::kAhead][2];
+    auto issue_w = [&](uint32_t (&w)[2]) {  // the next block's two words
+        w[0] = __builtin_amdgcn_raw_buffer_load_b32(rw, woff, 0, 0);
+        w[1] = __builtin_amdgcn_raw_buffer_load_b32(rw, woff, t.wq_stride, 0);
+        woff += wstep;
+    };
+#pragma unroll
+    for (int j = 0; j < G::kAhead; ++j) issue_w(ring[j]);
+
+    store_round(s_buf[0]);
+    load_round(G::kBlocks);
+    __syncthreads();
+
+    // Three stages over groups of kSub blocks: activation fragments read from
+    // LDS one group ahead of their MFMAs, the scales with them, and a group's
+    // dots scaled while the next group's MFMAs run.  The first group scaled is
+    // a zero one (+0 terms).
+    float acc[RT][4] = {};
+    const v4i cin = {kDotBiasBits, kDotBiasBits, kDotBiasBits, kDotBiasBits};
+    long frag[2][RT][G::kSub];
+    v4i dots[2][RT][G::kSub];
+    int da[2][RT];  // lane (kg, 4 j + e): the scale of row 4 kg + e and the group's block j
+    float2 dw[2][G::kSub];
+#pragma unroll
+    for (int j = 0; j < G::kSub; ++j) {
+#pragma unroll
+        for (int r = 0; r < RT; ++r) dots[1][r][j] = cin;
+        dw[1][j] = make_float2(0.0f, 0.0f);
+    }
+#pragma unroll
+    for (int r = 0; r < RT; ++r) da[1][r] = 0;
+    auto read_frags = [&](const typename G::Buf &s, int b, long (&f)[RT][G::kSub]) {
+#pragma unroll
+        for (int j = 0; j < G::kSub; ++j)
+#pragma unroll
+            for (int r = 0; r < RT; ++r)
+                f[r][j] = *reinterpret_cast<const long *>(s.a + (b + j) * G::kPitch + r * 512 + lane * 8);
+    };
+    // Output row e of block j: its activation scale is broadcast from lane
+    // 4 j + e of each row of 16 lanes (DPP row_newbcast, folded into the
+    // multiply).
+    auto scale_one = [&](int p, auto jc, auto ec) {
+        constexpr int j = decltype(jc)::value, e = decltype(ec)::value;
+#pragma unroll
+        for (int r = 0; r < RT; ++r) {
+            const float d = __int_as_float(__builtin_amdgcn_update_dpp(0, da[p][r], 0x150 + 4 * j + e, 0xF, 0xF, true));
+            acc[r][e] = acc[r][e] + fmaf(__int_as_float(dots[p][r][j][e]), dw[p][j].x, dw[p][j].y) * d;
+        }
+    };
+    auto scale = [&](int p) {
+        auto block = [&](auto jc) {
+            scale_one(p, jc, std::integral_constant<int, 0>{});
+            scale_one(p, jc, std::integral_constant<int, 1>{});
+            scale_one(p, jc, std::integral_constant<int, 2>{});
+            scale_one(p, jc, std::integral_constant<int, 3>{});
+        };
+        block(std::integral_constant<int, 0>{});
+        block(std::integral_constant<int, 1>{});
+        block(std::integral_constant<int, 2>{});
+        block(std::integral_constant<int, 3>{});
+    };
+    for (int c0 = 0, buf = 0; c0 < t.blocks; c0 += G::kBlocks, buf ^= 1) {
+        const typename G::Buf &s = s_buf[buf];
+        // Whole groups of kAhead blocks; blocks past K have zero scales, so
+        // their terms are +0 and change nothing.
+        const int nb = min(G::kBlocks, t.blocks - c0);
+        read_frags(s, 0, frag[0]);
+        for (int g = 0; g < nb; g += G::kAhead) {
+#pragma unroll
+            for (int q = 0; q < G::kAhead / G::kSub; ++q) {
+                const int b = g + q * G::kSub, p = q & 1;
+                read_frags(s, min(b + G::kSub, G::kBlocks - G::kSub), frag[p ^ 1]);
+#pragma unroll
+                for (int j = 0; j < G::kSub; ++j) dw[p][j] = s.dw[b + j][wave * 16 + l16];
+#pragma unroll
+                for (int r = 0; r < RT; ++r) da[p][r] = __float_as_int(s.da[b / G::kSub][r * 64 + lane]);
+                __builtin_amdgcn_sched_barrier(0);  // keep the reads ahead of their use
+#pragma unroll
+                for (int j = 0; j < G::kSub; ++j) {
+                    uint32_t(&w)[2] = ring[q * G::kSub + j];
+#pragma unroll
+                    for (int r = 0; r < RT; ++r)
+                        dots[p][r][j] = __builtin_amdgcn_mfma_i32_16x16x32_i8(
+                            frag[p][r][j], static_cast<long>((static_cast<uint64_t>(w[1]) << 32) | w[0]), cin, 0, 0, 0);
+                    issue_w(w);
+                }
+                scale(p ^ 1);
+                // The scaling stays here: sunk past the next group's reads it
+                // would hold every group's dots and scales in registers.
+#pragma unroll
+                for (int r = 0; r < RT; ++r)
+                    asm volatile("" : "+v"(acc[r][0]), "+v"(acc[r][1]), "+v"(acc[r][2]), "+v"(acc[r][3]));
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        // The other buffer was last read a round ago, before the previous barrier.
+        store_round(s_buf[buf ^ 1]);
+        load_round(c0 + 2 * G::kBlocks);
+        __syncthreads();
+    }
+    scale(1);  // a round ends on an odd group
+    const bool exact = __syncthreads_or(!finite);
+    if (!b_ok) return;
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int m = m0 + r * 16 + kg * 4 + e;
+            if (m < t.m)
+                reinterpret_cast<float *>(reinterpret_cast<uint8_t *>(t.y) + static_cast<size_t>(m) * t.y_stride)[t.ocol0 + bn] =
+                    exact ? exact_output_split(t, m, bn) : acc[r][e];
         }
 }
 
@@ -639,6 +874,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, SEL
         }
 }
 
+// The running weight offset of q4_0_tiled16_kernel stays below 2^32: it ends
+// one ring and one staged round past K, from a base of at most the extent.
+bool split16_supported(const TiledArgs &t) {
+    return t.cs == nullptr && t.w_extent + (2ull * Split16<1>::kBlocks + Split16<1>::kAhead + t.blocks) * 8 * t.wq_stride < (1ull << 32);
+}
+
 int launch_tiled(const TiledArgs &t, bool native, hipStream_t stream) {
     const dim3 grid((t.n + kTile - 1) / kTile, (t.m + kTile - 1) / kTile, 1);
     if (grid.y > 65535u) return fail(QXT_INVALID_ARGUMENT, "q4_0 tiled linear: too many rows");
@@ -653,6 +894,22 @@ int launch_tiled(const TiledArgs &t, bool native, hipStream_t stream) {
         return launch("q4_0_tiled_kernel", q4_0_staged_kernel<false>, grid, dim3(kThreads), 0, stream, t);
     }
     if (t.cs != nullptr) return launch("q4_0_tiled_kernel", q4_0_tiled_kernel<true>, grid, dim3(kThreads), 0, stream, t);
+    if (split16_supported(t)) {
+        // Sixteen-row tiles up to two waves per SIMD (eight per CU), where the
+        // chain of blocks per wave sets the time (M = 100, K = N = 4096, 1792
+        // waves: 16.4 us against 18.8 with 32-row and 27.3 with 64-row tiles;
+        // M = 160, 2560 waves: 25.0, 24.2 and 28.0); 32-row tiles past that
+        // from K = 2048, where a workgroup's first staged round is paid for
+        // (K = 2048, M = 512, N = 4096: 28.9 against 29.4 us with 64-row tiles;
+        // K = 1024: 17.9 against 16.6; K = 512, N = 8000: 25.1 against 20.8).
+        const long waves = 4L * grid.x * ((t.m + 15) / 16);
+        if (waves <= 8L * compute_units())
+            return launch("q4_0_tiled_kernel", q4_0_tiled16_kernel<1>, dim3(grid.x, (t.m + 15) / 16), dim3(kThreads),
+                          0, stream, t);
+        if (t.blocks >= 64 && (t.m + 31) / 32 <= 65535)
+            return launch("q4_0_tiled_kernel", q4_0_tiled16_kernel<2>, dim3(grid.x, (t.m + 31) / 32), dim3(kThreads),
+                          0, stream, t);
+    }
     return launch("q4_0_tiled_kernel", q4_0_tiled_kernel<false>, grid, dim3(kThreads), 0, stream, t);
 }
 
