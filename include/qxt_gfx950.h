@@ -194,8 +194,9 @@ int qxt_ggml_geglu_q8_0_split(const float *gate, size_t gate_row_stride, const f
  * wc = weight_column_start + j, for r < rows, j < column_count.
  * activation: Q8_0 u8 [rows, blocks, 34]; weight: Q4_0 u8 [>= wc+1, blocks, 18].
  * Writes only destination[:, output_column_start : +column_count].  rows >= 16 run on the
- * int8 matrix cores (one MFMA per 32 x 32 outputs and block); 4 to 15 rows with blocks / 8
- * dividing 16 (K <= 4096) on v_mfma_i32_4x4x4_16b_i8; other shapes on v_dot4.
+ * int8 matrix cores (one MFMA per 32 x 32 outputs and block); 2 to 15
+ * rows with blocks % 8 == 0 run on 16 x 16 x 32 or 4 x 4 x 4 matrix-core tiles or,
+ * like one row, on v_dot4, by shape.
  * Replaces GGML_Q4_0_Q8_0_LINEAR_KERNEL (src/qpu_xla/kernels/ggml_q4_0.py:783-841)
  * and the device work of qpu_llama_q4_0_linear_submit (qpu_llama_q4_0.h:72-75). */
 int qxt_ggml_q4_0_q8_0_linear(const void *activation, size_t activation_row_stride,
@@ -227,9 +228,8 @@ int qxt_q4_0_pack_lanes(const void *weight, size_t weight_row_stride, void *pack
 
 /* qxt_ggml_q4_0_q8_0_linear over a lane-layout weight of `weight_columns`
  * columns (weight_column_start + column_count <= weight_columns); same
- * result bit for bit.  Four or more rows with blocks / 8 dividing 16 (K <= 4096)
- * run on v_mfma_i32_4x4x4_16b_i8 (four rows x four columns per 4-lane block);
- * other shapes on v_dot4. */
+ * result bit for bit.  Two or more rows run on matrix-core tiles or
+ * v_dot4, by shape, as for qxt_ggml_q4_0_q8_0_linear. */
 int qxt_ggml_q4_0_q8_0_linear_lanes(const void *activation, size_t activation_row_stride,
                                     const void *packed_weight, uint32_t weight_columns,
                                     float *destination, size_t destination_row_stride,
@@ -286,10 +286,10 @@ int qxt_ggml_q8_0_q8_0_linear(const void *activation, size_t activation_row_stri
 
 /* One linear of a Q4_0 batch.  Exactly one of `x` (fp32 rows [rows, blocks*32]
  * with 16-byte aligned rows, quantised to Q8_0 by the rule of qxt_quantize_q8_0:
- * in a pre-pass launch of the batch when the batch has more than 1024 work
- * items, else by every workgroup that reads them) and `activation` (native
- * Q8_0 blocks) is non-NULL; the
- * other fields mean what they mean for qxt_ggml_q4_0_q8_0_linear.  Batched
+ * by every workgroup that reads them in a batch of few columns, else in a
+ * pre-pass launch of the batch) and `activation` (native Q8_0 blocks) is
+ * non-NULL; the other fields mean what they mean for
+ * qxt_ggml_q4_0_q8_0_linear.  Batched
  * tasks need rows <= 4, blocks % 8 == 0 and 16-byte aligned weight rows.
  * weight_layout QXT_Q4_0_LAYOUT_LANES: `weight` is the base of a
  * qxt_q4_0_pack_lanes matrix and weight_row_stride is ignored. */
@@ -321,7 +321,7 @@ typedef struct qxt_q4_0_batch qxt_q4_0_batch;
 int qxt_q4_0_batch_prepare(const qxt_q4_0_task *tasks, uint32_t count, qxt_q4_0_batch **batch);
 
 /* Enqueue the whole batch on `stream`: the Q8_0 pre-pass (when a task has fp32
- * rows and the batch has more than 1024 work items) and the batch grid;
+ * rows that the batch grid does not quantise itself) and the batch grid;
  * graph-capturable.
  * Replaces qpu_llama_q4_0_linear_submit (qpu_llama_q4_0.h:72-75). */
 int qxt_q4_0_batch_launch(const qxt_q4_0_batch *batch, void *stream);

@@ -49,6 +49,7 @@ HIPCC_FLAGS = [
 SOURCE_FLAGS = {
     "qxt_q4_0_tiled.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "qxt_q4_0.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "qxt_q4_0_rows.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }
 
 

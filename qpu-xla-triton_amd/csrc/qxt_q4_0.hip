@@ -52,7 +52,7 @@
 #include <utility>
 #include <vector>
 
-#include "qxt_common.h"
+#include "qxt_q4_0.h"
 
 namespace qxt {
 namespace {
@@ -61,45 +61,6 @@ constexpr int kThreads = 256;
 constexpr size_t kMaxLds = 64 * 1024;       // LDS a workgroup may use to stage its activation rows
 constexpr size_t kMaxLdsWide = 160 * 1024;  // gfx950 LDS per workgroup: wide single-linear tiles
 
-struct Q4Task {
-    const float *x;        // fp32 rows quantised to Q8_0 in the workgroup, or nullptr
-    size_t x_stride;
-    const uint8_t *act;    // native Q8_0 blocks [rows, blocks, 34] (when x is nullptr)
-    const uint8_t *w;      // Q4_0 blocks [N, blocks, 18]
-    float *y;              // fp32 output
-    int32_t *dots;         // debug: int32 block dots [rows, ncols, blocks]
-    size_t act_stride, w_stride, y_stride;  // row strides in bytes
-    int rows, blocks, wcol0, ocol0, ncols, cpw;
-    int lanes;             // weight in the lane-interleaved layout (w = packed matrix base)
-};
-
-constexpr int kLaneGroup = 64;                      // units per lane group
-constexpr int kUnitBytes = 144;                     // 8 Q4_0 blocks of one column
-constexpr int kGroupBytes = kLaneGroup * kUnitBytes;  // 9216
-
-struct Q4Item {
-    int task;
-    int col_base;
-    int ncols;  // columns of this work item (<= the task's cpw)
-};
-
-typedef unsigned int v4u __attribute__((ext_vector_type(4)));
-
-// Batch kernels read their tensor pointers from a device table, so the
-// compiler cannot tell they address global memory and would emit FLAT
-// loads.  A FLAT load also counts against the LDS counter, which turns every
-// later wait for an LDS access into a wait for all outstanding weight loads
-// (activation staging then starts only after the weights have landed).
-// Every tensor access goes through a global-address-space pointer instead.
-#define QXT_GLOBAL __attribute__((address_space(1)))
-template <typename T>
-__device__ __forceinline__ const QXT_GLOBAL T *global_in(const void *p) {
-    return (const QXT_GLOBAL T *)p;
-}
-template <typename T>
-__device__ __forceinline__ QXT_GLOBAL T *global_out(void *p) {
-    return (QXT_GLOBAL T *)p;
-}
 __device__ __forceinline__ float4 load_float4(const void *p) {
     const v4u raw = *global_in<v4u>(p);
     return make_float4(__uint_as_float(raw[0]), __uint_as_float(raw[1]), __uint_as_float(raw[2]),
@@ -126,23 +87,6 @@ struct Q4Lds {
 // on distinct banks.
 __device__ __forceinline__ int aq_index(int b, int j) { return b * 8 + (b >> 3) * 4 + j; }
 __device__ __forceinline__ int ad_index(int b) { return 2 * (b + (b >> 3)); }
-
-// Block i (0..7) of a 144-byte unit held as 36 little-endian words: returns
-// the fp16 scale bits and the 4 words of packed nibbles.
-template <int I>
-__device__ __forceinline__ void unit_block(const uint32_t (&d)[36], uint32_t &sbits, uint32_t (&qs)[4]) {
-    if constexpr ((I & 1) == 0) {
-        constexpr int k = 9 * I / 2;  // block starts word-aligned: d then nibbles at +2 bytes
-        sbits = d[k] & 0xFFFFu;
-#pragma unroll
-        for (int t = 0; t < 4; ++t) qs[t] = __builtin_amdgcn_alignbyte(d[k + t + 1], d[k + t], 2);
-    } else {
-        constexpr int k = (9 * I - 1) / 2;  // block starts at a half word: nibbles word-aligned
-        sbits = d[k] >> 16;
-#pragma unroll
-        for (int t = 0; t < 4; ++t) qs[t] = d[k + 1 + t];
-    }
-}
 
 // Exact int32 dot of one Q4_0 block (packed nibbles qs) with one Q8_0 block
 // (activation words a0, a1 and their element sum asum).
@@ -430,12 +374,6 @@ __device__ __forceinline__ void stage_q8_row(const Q4Task &t, const Q8RowRegs<NT
         store_scale_sum<false>(ad, geo, 0, b, half_bits_to_float(a.h[i][0]), sum);
     }
 }
-
-// Weight layout of a kernel instantiation: native rows, lane layout, or
-// either (read from the task).  Separate instantiations keep the lane
-// layout's non-temporal loads from being merged with the native rows'
-// ordinary loads of the other branch.
-enum WeightLayout { kNativeRows = 0, kLaneLayout = 1, kEitherLayout = 2 };
 
 // CLAMP: every lane issues its loads, a lane past the tile re-reading the
 // tile's last unit (its registers are never used).  The loads are then
@@ -1048,18 +986,6 @@ __global__ __launch_bounds__(NT) void q4_0_batch_kernel(const Q4Task *__restrict
     batch_item_any<MR, U, LAYOUT, PC, S, NT>(tasks[item.task], item.col_base, item.ncols);
 }
 
-// A batch of at most kArgTasks tasks travels in the kernel arguments: each
-// workgroup finds its task and column tile from its index, without the two
-// dependent reads of a device table (item, then task) before its first
-// weight or activation request.  Task j's items start at first_item[j]
-// (INT_MAX past the last task) and are its column tiles of cpw columns in
-// order.
-constexpr int kArgTasks = 4;
-struct Q4ArgBatch {
-    int first_item[kArgTasks];
-    Q4Task task[kArgTasks];
-};
-
 template <int MR, int U, int LAYOUT, int PC, int S = 1, int NT = kThreads>
 __global__ __launch_bounds__(NT) void q4_0_arg_batch_kernel(Q4ArgBatch a) {
     const int i = static_cast<int>(blockIdx.x);
@@ -1522,6 +1448,8 @@ struct qxt_q4_0_batch {
     int split = 1;     // waves per unit (one-row prefetch batches of narrow items)
     int threads = kThreads;  // 256, or 512 / 1024 for split prefetch batches
     size_t lds = 0;
+    bool rows = false;     // the row-tile kernels (tasks of two to four rows)
+    bool rows_fp32 = false;  // they quantise fp32 rows themselves
     bool in_args = false;  // tasks and items travel in the kernel arguments
     Q4ArgBatch args{};
 };
@@ -1606,6 +1534,20 @@ int qxt_ggml_q4_0_q8_0_linear(const void *activation, size_t activation_row_stri
         return q4_0_tiled_native(activation, activation_row_stride, weight, weight_row_stride, destination,
                                  destination_row_stride, rows, blocks, weight_column_start, output_column_start,
                                  column_count, as_stream(stream));
+    Q4Task t{};
+    t.act = static_cast<const uint8_t *>(activation);
+    t.act_stride = activation_row_stride;
+    t.w = static_cast<const uint8_t *>(weight);
+    t.w_stride = weight_row_stride;
+    t.y = destination;
+    t.y_stride = destination_row_stride;
+    t.rows = static_cast<int>(rows);
+    t.blocks = static_cast<int>(blocks);
+    t.wcol0 = static_cast<int>(weight_column_start);
+    t.ocol0 = static_cast<int>(output_column_start);
+    t.ncols = static_cast<int>(column_count);
+    rc = q4_0_rows_linear(t, as_stream(stream));
+    if (rc != QXT_CAPABILITY_MISSING) return rc;
     // Long rows spread their blocks over the lanes instead: more than 64
     // blocks with two or more activation rows (128 for four rows over fewer
     // than 8192 columns), more than 256 with one (measured on MI355X, event-timed: M=4
@@ -1627,18 +1569,6 @@ int qxt_ggml_q4_0_q8_0_linear(const void *activation, size_t activation_row_stri
                                 column_count, as_stream(stream));
         if (rc != QXT_CAPABILITY_MISSING) return rc;
     }
-    Q4Task t{};
-    t.act = static_cast<const uint8_t *>(activation);
-    t.act_stride = activation_row_stride;
-    t.w = static_cast<const uint8_t *>(weight);
-    t.w_stride = weight_row_stride;
-    t.y = destination;
-    t.y_stride = destination_row_stride;
-    t.rows = static_cast<int>(rows);
-    t.blocks = static_cast<int>(blocks);
-    t.wcol0 = static_cast<int>(weight_column_start);
-    t.ocol0 = static_cast<int>(output_column_start);
-    t.ncols = static_cast<int>(column_count);
     return dispatch_single<false>(t, as_stream(stream));
 }
 
@@ -1698,6 +1628,8 @@ int qxt_ggml_q4_0_q8_0_linear_lanes(const void *activation, size_t activation_ro
     t.wcol0 = static_cast<int>(weight_column_start);
     t.ocol0 = static_cast<int>(output_column_start);
     t.ncols = static_cast<int>(column_count);
+    rc = q4_0_rows_linear(t, as_stream(stream));
+    if (rc != QXT_CAPABILITY_MISSING) return rc;
     return dispatch_single<false>(t, as_stream(stream));
 }
 
@@ -1830,6 +1762,15 @@ int qxt_q4_0_batch_prepare(const qxt_q4_0_task *tasks, uint32_t count, qxt_q4_0_
     // its weights and quantises it while they are in flight.  A batch whose
     // tiles were narrowed (too few columns to fill the chip) runs it with
     // kPrefetchUnits units per thread, its tiles planned for that.
+    // Batches with tasks of two to four rows run the row-tile kernels, which
+    // quantise fp32 rows themselves when every task of a small batch gives
+    // them and read the pre-pass's Q8_0 rows otherwise.
+    bool row_tiles = mr != 1;
+    for (uint32_t i = 0; i < count && row_tiles; ++i) {
+        Q4Task t = host[i];
+        t.x = nullptr;
+        row_tiles = q4_0_rows_batch_supported(t);
+    }
     bool prefetch_candidate = mr == 1;
     for (uint32_t i = 0; i < count && prefetch_candidate; ++i) prefetch_candidate = prefetch_chunks(host[i]) > 0;
     const bool small = static_cast<size_t>(planned) <= kFusedQuantItems;
@@ -1837,7 +1778,14 @@ int qxt_q4_0_batch_prepare(const qxt_q4_0_task *tasks, uint32_t count, qxt_q4_0_
     // Every other small batch quantises its fp32 rows inside each workgroup
     // too (an L2-resident re-read per workgroup) rather than waiting for a
     // separate pre-pass launch; larger ones run the pre-pass.
-    const bool fused = small || prefetch_candidate;
+    // (Up to eight column tiles per CU: the 16-stage step of four rows over
+    // K = 4096 / 11008 layers, fused 239, pre-pass 268 us; whole-step batches of
+    // thousands of tiles, pre-pass 134, fused 154 us.)
+    uint64_t row_tile_count = 0;
+    for (uint32_t i = 0; i < count; ++i) row_tile_count += (static_cast<uint64_t>(host[i].ncols) + 15) / 16;
+    const bool rows_fp32 =
+        row_tiles && jobs.size() == count && row_tile_count <= 8ull * static_cast<uint64_t>(compute_units());
+    const bool fused = row_tiles ? rows_fp32 : small || prefetch_candidate;
     const bool narrowed = max_cpw < (1 << 30);
     const int upt = prefetch_candidate && narrowed ? kPrefetchUnits : units_per_thread(mr);
     if (upt != units_per_thread(mr)) {
@@ -1873,8 +1821,16 @@ int qxt_q4_0_batch_prepare(const qxt_q4_0_task *tasks, uint32_t count, qxt_q4_0_
     }
     size_t lds = 0;
     std::vector<Q4Item> items;
-    const int64_t final_items = plan_items(upt, max_cpw, &items, &lds);
-    if (final_items < 0) return static_cast<int>(-final_items);
+    int threads = kThreads;
+    if (row_tiles) {
+        threads = q4_0_rows_plan(host.data(), count, &lds);
+        for (uint32_t i = 0; i < count; ++i)
+            for (int c = 0; c < host[i].ncols; c += host[i].cpw)
+                items.push_back({static_cast<int>(i), c, std::min(host[i].cpw, host[i].ncols - c)});
+    } else {
+        const int64_t final_items = plan_items(upt, max_cpw, &items, &lds);
+        if (final_items < 0) return static_cast<int>(-final_items);
+    }
     if (fused) {
         jobs.clear();
         job_task.clear();
@@ -1935,6 +1891,9 @@ int qxt_q4_0_batch_prepare(const qxt_q4_0_task *tasks, uint32_t count, qxt_q4_0_
     batch->chunk_count = static_cast<uint32_t>(chunks.size());
     batch->grid = static_cast<uint32_t>(items.size());
     batch->mr = mr;
+    batch->rows = row_tiles;
+    batch->rows_fp32 = rows_fp32;
+    batch->threads = threads;
     batch->layout = layout;
     // The prefetch kernel runs exactly the batches planned for it.
     batch->prefetch = 0;
@@ -1997,6 +1956,9 @@ int qxt_q4_0_batch_launch(const qxt_q4_0_batch *batch, void *stream) {
                     as_stream(stream), batch->jobs, batch->chunks);
         if (rc != QXT_OK) return rc;
     }
+    if (batch->rows)
+        return q4_0_rows_batch(batch->in_args ? &batch->args : nullptr, batch->tasks, batch->items, batch->grid,
+                               batch->threads, batch->lds, batch->layout, batch->rows_fp32, as_stream(stream));
     const BatchKernel kernel =
         batch_kernel(batch->mr, batch->layout, batch->prefetch, batch->upt, batch->split, batch->threads);
     const dim3 block(batch->threads);

@@ -59,3 +59,105 @@ def test_split_plane_32_row_tiles_redo_a_tile_with_a_non_finite_scale() -> None:
     some = np.arange(4960, 5060)
     with np.errstate(invalid="ignore"):
         np.testing.assert_array_equal(out[:, some], oracle.q4_0_q8_0_reference(act, wt[some]))
+
+
+def _check_linear(layout: str, rows: int, blocks: int, n: int, wcol0: int, ncols: int, act=None, wt=None) -> None:
+    if act is None:
+        act, wt = _operands(rows * 100003 + blocks * 17 + n, rows, blocks, n)
+    out = torch.full((rows, ncols + 9), -77.0, device="cuda")
+    weight = q4.pack_ggml_q4_0_lane_weights(dev(wt)) if layout == "lanes" else dev(wt)
+    linear = q4.ggml_q4_0_q8_0_lane_linear if layout == "lanes" else q4.ggml_q4_0_q8_0_linear
+    linear(dev(act), weight, out, weight_column_start=wcol0, output_column_start=5, column_count=ncols)
+    got = out.cpu().numpy()
+    np.testing.assert_array_equal(got[:, :5], -77.0)
+    np.testing.assert_array_equal(got[:, 5 + ncols:], -77.0)
+    some = np.unique(np.concatenate([np.arange(min(ncols, 96)), np.arange(max(0, ncols - 96), ncols)]))
+    np.testing.assert_array_equal(got[:, 5 + some], oracle.q4_0_q8_0_reference(act, wt[wcol0 + some]))
+
+
+@pytest.mark.parametrize("layout", ["lanes", "native"])
+@pytest.mark.parametrize("rows,blocks,n,wcol0,ncols", [
+    (2, 8, 33, 0, 33),        # one unit, ragged columns
+    (3, 16, 40, 7, 20),       # one half-unit chunk of four lanes, a column range
+    (4, 24, 17, 1, 16),       # one unit past a chunk
+    (5, 40, 100, 0, 100),     # two rows per lane, or two row groups
+    (6, 32, 6000, 0, 6000),   # more tiles than CUs: every row in one group
+    (8, 64, 5632, 3, 5629),
+    (9, 72, 300, 0, 300),     # units no power of two
+    (12, 48, 4200, 0, 4200),  # three rows per lane
+    (15, 136, 2048, 0, 2048),
+    (13, 56, 8300, 0, 8300),  # four rows per lane, whole-unit chunks
+    (5, 128, 9000, 2, 8990),  # several tiles per workgroup
+    (10, 264, 4112, 0, 4112),  # several chunks per wave
+    (15, 344, 4112, 16, 4096),  # rows in groups (LDS)
+    (4, 520, 4112, 0, 4112),  # three chunks per wave, four rows
+])
+def test_row_tile_linear_bit_exact(layout: str, rows: int, blocks: int, n: int, wcol0: int, ncols: int) -> None:
+    _check_linear(layout, rows, blocks, n, wcol0, ncols)
+
+
+@pytest.mark.parametrize("layout", ["lanes", "native"])
+def test_row_tile_linear_non_finite_and_extreme_scales_bit_exact(layout: str) -> None:
+    # dw enters as dw / 16 times 16 dots: subnormal, largest, infinite and NaN fp16 scales.
+    act, wt = _operands(11, 6, 24, 64)
+    bits = np.array([0x0001, 0x03FF, 0x0400, 0x7BFF, 0xFBFF, 0x7C00, 0xFC00, 0x7E00, 0x0000, 0x8000], dtype=np.uint16)
+    wt.reshape(-1, 18)[:: 7, :2] = np.resize(bits, (wt.reshape(-1, 18)[:: 7].shape[0],)).view(np.uint8).reshape(-1, 2)
+    act.reshape(-1, 34)[:: 5, :2] = np.resize(bits, (act.reshape(-1, 34)[:: 5].shape[0],)).view(np.uint8).reshape(-1, 2)
+    with np.errstate(all="ignore"):
+        _check_linear(layout, 6, 24, 64, 0, 64, act, wt)
+
+
+def test_row_tile_linear_unaligned_activation_takes_the_general_kernel() -> None:
+    act, wt = _operands(12, 5, 64, 80)
+    raw = torch.zeros(act.size + 2, dtype=torch.uint8, device="cuda")
+    raw[2:] = dev(act).flatten()
+    shifted = raw[2:].view(act.shape)  # two bytes past a word
+    assert shifted.data_ptr() % 4 == 2
+    out = q4.ggml_q4_0_q8_0_linear(shifted, dev(wt)).cpu().numpy()
+    np.testing.assert_array_equal(out, oracle.q4_0_q8_0_reference(act, wt))
+
+
+@pytest.mark.parametrize("count", [2, 4, 7])  # kernel arguments up to four tasks, device tables past that
+@pytest.mark.parametrize("layouts", ["lanes", "native", "mixed"])
+def test_row_tile_batch_mixed_rows_lengths_and_activations_bit_exact(count: int, layouts: str) -> None:
+    rng = np.random.default_rng(count * 10 + len(layouts))
+    shapes = [(4, 64, 700), (1, 8, 16), (3, 176, 130), (2, 264, 50), (4, 40, 1), (2, 16, 4100), (1, 128, 33)][:count]
+    tasks, expected = [], []
+    for i, (rows, blocks, n) in enumerate(shapes):
+        x = rng.standard_normal((rows, blocks * 32), dtype=np.float32)
+        w = (rng.standard_normal((n, blocks * 32), dtype=np.float32) * np.float32(0.02)).astype(np.float32)
+        act, wt = oracle.quantize_q8_0_blocks(x), oracle.quantize_q4_0_blocks(w)
+        lanes = layouts == "lanes" or (layouts == "mixed" and i % 2 == 0)
+        task = {"weight": q4.pack_ggml_q4_0_lane_weights(dev(wt)) if lanes else dev(wt),
+                "destination": torch.full((rows, n + 3), -77.0, device="cuda"), "output_column_start": 2}
+        task["x" if i % 3 != 1 else "activation"] = dev(x) if i % 3 != 1 else dev(act)
+        tasks.append(task)
+        expected.append(oracle.q4_0_q8_0_reference(act, wt))
+    with q4.Q4_0LinearBatch(tasks) as batch:
+        for _ in range(2):
+            batch.launch()
+        torch.cuda.synchronize()
+        for task, want in zip(tasks, expected):
+            got = task["destination"].cpu().numpy()
+            np.testing.assert_array_equal(got[:, 2:-1], want)
+            np.testing.assert_array_equal(got[:, [0, 1, -1]], -77.0)
+
+
+def test_row_tile_batch_captured_and_replayed_reads_the_rows_of_each_replay() -> None:
+    act, wt = _operands(13, 4, 64, 300)
+    x = torch.zeros((4, 2048), device="cuda")
+    out = torch.zeros((4, 300), device="cuda")
+    with q4.Q4_0LinearBatch([{"x": x, "weight": dev(wt), "destination": out}]) as batch:
+        batch.launch()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            batch.launch()
+        rng = np.random.default_rng(14)
+        for _ in range(3):
+            rows = rng.standard_normal((4, 2048), dtype=np.float32)
+            x.copy_(torch.from_numpy(rows))
+            graph.replay()
+            torch.cuda.synchronize()
+            np.testing.assert_array_equal(
+                out.cpu().numpy(), oracle.q4_0_q8_0_reference(oracle.quantize_q8_0_blocks(rows), wt))
