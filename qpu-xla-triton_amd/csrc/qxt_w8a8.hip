@@ -78,9 +78,10 @@ struct StageRegs {
 
     __device__ __forceinline__ void load(const GemmArgs &args, __amdgpu_buffer_rsrc_t ra, __amdgpu_buffer_rsrc_t rb,
                                          int m0, int n0, int k0) {
+        const int tid = threadIdx.x % kThreads;
 #pragma unroll
         for (int i = 0; i < A_CHUNKS; ++i) {
-            const int c = threadIdx.x + i * kThreads;
+            const int c = tid + i * kThreads;
             const int row = c / CPR, kc = c % CPR;
             const int gm = m0 + row, gk = k0 + kc * 16;
             const uint32_t off = (gm < args.m && gk < args.k) ? static_cast<uint32_t>(gm) * args.lda + gk : kOutOfRange;
@@ -88,7 +89,7 @@ struct StageRegs {
         }
 #pragma unroll
         for (int i = 0; i < B_CHUNKS; ++i) {
-            const int c = threadIdx.x + i * kThreads;
+            const int c = tid + i * kThreads;
             uint32_t off;
             if constexpr (!K4N) {
                 const int row = c / CPR, kc = c % CPR;
@@ -105,15 +106,16 @@ struct StageRegs {
     }
 
     __device__ __forceinline__ void store(uint8_t *As, uint8_t *Bs) const {
+        const int tid = threadIdx.x % kThreads;
         constexpr int ROW = BKT + 16;
 #pragma unroll
         for (int i = 0; i < A_CHUNKS; ++i) {
-            const int c = threadIdx.x + i * kThreads;
+            const int c = tid + i * kThreads;
             *reinterpret_cast<v4u *>(As + (c / CPR) * ROW + (c % CPR) * 16) = a[i];
         }
 #pragma unroll
         for (int i = 0; i < B_CHUNKS; ++i) {
-            const int c = threadIdx.x + i * kThreads;
+            const int c = tid + i * kThreads;
             if constexpr (!K4N) {
                 *reinterpret_cast<v4u *>(Bs + (c / CPR) * ROW + (c % CPR) * 16) = b[i];
             } else {
@@ -299,20 +301,27 @@ constexpr int kEpilogueLds = 128 * 1024 + 3 * 256 * 4;
 // loads are issued before the current stage's MFMAs and written to the other
 // buffer after them, one barrier per stage.  Within a stage the fragments of
 // the next 32-deep k step are read from LDS while the current step's MFMAs run.
-template <int BM, int BN, int BKT, int DEPTH, int STORE_KS, bool K4N, int EPI>
-__global__ __launch_bounds__(kThreads) void w8a8_gemm_kernel(GemmArgs args) {
+//
+// KS > 1: KS groups of four waves share the tile, group g taking K stages g,
+// g + KS, ... with buffers of its own; the groups' exact int32 sums are added
+// through LDS at the end.
+template <int BM, int BN, int BKT, int DEPTH, int STORE_KS, int KS, bool K4N, int EPI>
+__global__ __launch_bounds__(KS * kThreads) void w8a8_gemm_kernel(GemmArgs args) {
     constexpr int ROW = BKT + 16;
     constexpr int STAGE = (BM + BN) * ROW;
     constexpr int KSTEPS = BKT / 32;
     static_assert(KSTEPS % 2 == 0, "fragment double buffer assumes an even number of k steps");
-    static_assert(DEPTH == 1 || DEPTH == 2, "one or two register stages in flight");
+    static_assert(DEPTH >= 1, "register stages in flight");
     static_assert(STORE_KS >= 0 && STORE_KS < KSTEPS, "store step inside the stage");
-    __shared__ __attribute__((aligned(16))) uint8_t smem[2 * STAGE];
+    static_assert((KS - 1) * BM * BN * 4 + 3 * 256 * 4 <= KS * 2 * STAGE, "the partial sums reuse the operand buffers");
+    __shared__ __attribute__((aligned(16))) uint8_t shared[KS * 2 * STAGE];
+    const int group = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kThreads));
+    uint8_t *const smem = shared + group * 2 * STAGE;
 
     constexpr int WM = BM / 2, WN = BN / 2;    // per-wave sub-tile
     constexpr int TM = WM / 32, TN = WN / 32;  // 32x32 blocks per wave
     const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
+    const int wave = (threadIdx.x >> 6) & 3;
     const int wm = wave >> 1, wn = wave & 1;
     const int m0 = blockIdx.y * BM;
     const int n0 = blockIdx.x * BN;
@@ -338,15 +347,16 @@ __global__ __launch_bounds__(kThreads) void w8a8_gemm_kernel(GemmArgs args) {
         for (int j = 0; j < TN; ++j) bf[buf][j] = *reinterpret_cast<const v4i *>(Bs + b_lane + j * 32 * ROW + kk);
     };
 
-    // DEPTH register stages in flight.  DEPTH == 1: stage s+1 is loaded at the
-    // start of stage s and written to LDS in k step STORE_KS of stage s.
-    // DEPTH == 2: stage s+2 is loaded at the start of stage s while stage s+1
-    // (loaded a full stage earlier) is written in k step STORE_KS.
-    const int stages = (args.k + BKT - 1) / BKT;
+    // DEPTH register stages in flight: stage s + DEPTH is loaded at the start
+    // of stage s while stage s + 1 (loaded DEPTH - 1 stages earlier; for
+    // DEPTH == 1 just now) is written to LDS in k step STORE_KS.
+    const int stages = (args.k + KS * BKT - 1) / (KS * BKT);  // of this group (past K: zeros)
+    const int k_first = group * BKT;
     StageRegs<BM, BN, BKT, K4N> regs[DEPTH];
-    regs[0].load(args, ra, rb, m0, n0, 0);
+    regs[0].load(args, ra, rb, m0, n0, k_first);
     regs[0].store(smem, smem + BM * ROW);
-    if constexpr (DEPTH == 2) regs[1].load(args, ra, rb, m0, n0, BKT);
+#pragma unroll
+    for (int d = 1; d < DEPTH; ++d) regs[d].load(args, ra, rb, m0, n0, k_first + d * KS * BKT);
     __syncthreads();
     read_frags(smem, smem + BM * ROW, 0, 0);
 
@@ -357,7 +367,7 @@ __global__ __launch_bounds__(kThreads) void w8a8_gemm_kernel(GemmArgs args) {
         const uint8_t *As = smem + (s & 1) * STAGE;
         const uint8_t *Bs = As + BM * ROW;
         uint8_t *next = smem + ((s + 1) & 1) * STAGE;
-        prefetch.load(args, ra, rb, m0, n0, (s + DEPTH) * BKT);
+        prefetch.load(args, ra, rb, m0, n0, k_first + (s + DEPTH) * KS * BKT);
 #pragma unroll
         for (int ks = 0; ks < KSTEPS; ++ks) {
             // One scheduling region per k step: the TM*TN independent MFMAs of
@@ -387,21 +397,52 @@ __global__ __launch_bounds__(kThreads) void w8a8_gemm_kernel(GemmArgs args) {
         __syncthreads();
         read_frags(next, next + BM * ROW, 0, 0);
     };
-    if constexpr (DEPTH == 1) {
-        for (int s = 0; s < stages; ++s) stage_body(s, regs[0], regs[0]);
-    } else {
-        int s = 0;
-        for (; s + 1 < stages; s += 2) {
-            stage_body(s, regs[0], regs[1]);
-            stage_body(s + 1, regs[1], regs[0]);
-        }
-        if (s < stages) stage_body(s, regs[0], regs[1]);
-    }
+    int s = 0;
+    for (; s + DEPTH <= stages; s += DEPTH)
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d) stage_body(s + d, regs[d], regs[(d + 1) % DEPTH]);
+#pragma unroll
+    for (int d = 0; d + 1 < DEPTH; ++d)
+        if (s + d < stages) stage_body(s + d, regs[d], regs[d + 1]);
 
     __syncthreads();
-    stage_scales<BM, BN, EPI>(args, reinterpret_cast<float *>(smem), m0, n0);
-    store_tile<BM, BN, TM, TN, EPI>(args, acc, m0 + wm * WM, n0 + wn * WN, wm * WM, wn * WN, lane,
-                                    reinterpret_cast<const float *>(smem));
+    float *scales = reinterpret_cast<float *>(shared);
+    if constexpr (KS > 1) {
+        // Groups 1 .. KS - 1 leave their accumulators behind the scales, one
+        // 16-byte piece per lane and register quad.
+        v4i *parts = reinterpret_cast<v4i *>(shared + 3 * 256 * 4);
+        auto piece = [&](int g, int i, int j, int q) -> v4i & {
+            return parts[(((((g - 1) * 4 + wave) * TM + i) * TN + j) * 4 + q) * 64 + lane];
+        };
+        if (group > 0) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        piece(group, i, j, q) = v4i{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2],
+                                                    acc[i][j][4 * q + 3]};
+        }
+        stage_scales<BM, BN, EPI>(args, scales, m0, n0);
+        if constexpr (EPI == EPI_I32) __syncthreads();
+        if (group > 0) return;
+#pragma unroll
+        for (int g = 1; g < KS; ++g)
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const v4i v = piece(g, i, j, q);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) acc[i][j][4 * q + e] += v[e];
+                    }
+    } else {
+        stage_scales<BM, BN, EPI>(args, scales, m0, n0);
+    }
+    store_tile<BM, BN, TM, TN, EPI>(args, acc, m0 + wm * WM, n0 + wn * WN, wm * WM, wn * WN, lane, scales);
 }
 
 // ----------------------------------------------------------------------------
@@ -1023,17 +1064,17 @@ __global__ __launch_bounds__(kThreads) void dequantize_kernel(const int32_t *__r
 #define QXT_GEMM_STORE_KS 2
 #endif
 
-template <int BM, int BN, int BKT, int DEPTH, int STORE_KS, bool K4N>
+template <int BM, int BN, int BKT, int DEPTH, int STORE_KS, bool K4N, int KS = 1>
 int launch_gemm(GemmArgs args, int epi, uint32_t layout, hipStream_t stream) {
     args.a_bytes = static_cast<uint32_t>(static_cast<size_t>(args.m - 1) * args.lda + args.k);
     args.w_bytes = layout == QXT_W8A8_WEIGHT_K4N
                        ? static_cast<uint32_t>(static_cast<size_t>(args.k / 4 - 1) * args.ldw + args.n * 4)
                        : static_cast<uint32_t>(static_cast<size_t>(args.n - 1) * args.ldw + args.k);
     dim3 grid((args.n + BN - 1) / BN, (args.m + BM - 1) / BM, 1);
-    auto kernel = epi == EPI_I32        ? w8a8_gemm_kernel<BM, BN, BKT, DEPTH, STORE_KS, K4N, EPI_I32>
-                  : epi == EPI_DEQUANT ? w8a8_gemm_kernel<BM, BN, BKT, DEPTH, STORE_KS, K4N, EPI_DEQUANT>
-                                       : w8a8_gemm_kernel<BM, BN, BKT, DEPTH, STORE_KS, K4N, EPI_DEQUANT_BIAS>;
-    return launch("w8a8_gemm_kernel", kernel, grid, dim3(kThreads), 0, stream, args);
+    auto kernel = epi == EPI_I32        ? w8a8_gemm_kernel<BM, BN, BKT, DEPTH, STORE_KS, KS, K4N, EPI_I32>
+                  : epi == EPI_DEQUANT ? w8a8_gemm_kernel<BM, BN, BKT, DEPTH, STORE_KS, KS, K4N, EPI_DEQUANT>
+                                       : w8a8_gemm_kernel<BM, BN, BKT, DEPTH, STORE_KS, KS, K4N, EPI_DEQUANT_BIAS>;
+    return launch("w8a8_gemm_kernel", kernel, grid, dim3(KS * kThreads), 0, stream, args);
 }
 
 int launch_stream(const GemmArgs &args, int epi, hipStream_t stream) {
@@ -1208,6 +1249,46 @@ bool gemv_path(int m, int k) {
     return m <= kGemvMaxRows && static_cast<size_t>(rows) * k <= kGemvMaxLds;
 }
 
+// Tiles of problems too small for 256 x 256 ones.  What bounds them is what a CU
+// takes in from L2, measured at 55 to 61 bytes per ns with any of these tiles,
+// so the choice is the largest tile that still gives (nearly) every CU one, with
+// at least two K stages in flight in registers: one stage in flight left each
+// stage waiting for L2 (0.6 us at 64 x 64).  Two groups of four waves per tile
+// (KS = 2) where a CU holds one workgroup.
+// Measured on MI355X, GEMM alone, rotated weights, back to back (M x K x N, us;
+// before: 128 x 128 tiles from one tile per CU, else 64 x 64, one stage in
+// flight):
+//   128 x 128:  512 x 4096 x 14336 55.8 -> 46.5, 1024 x 4096 x 8192 53.2 -> 48.9;
+//               KS = 2: 1024 x 4096 x 4096 44.7 -> 26.9, 256 x 4096 x 14336 36.4 -> 27.2,
+//               256 x 4096 x 11008 (172 tiles) 32.9 -> 26.2; at 141 tiles 23.7
+//               against 21.7 with 64 x 64;
+//   128 x 64:   512 x 14336 x 4096 89.5 -> 51.7 (64 x 64: 62.3), 512 x 4096 x 4096
+//               27.2 -> 18.4; a second round of them (282 tiles) 28.3 against 21.7;
+//   64 x 64:    KS = 2, three stages: 48 x 4096 x 14336 29.1 -> 14.8, 128 x 14336 x
+//               4096 87.4 -> 34.4, 8 x 14336 x 4096 89.0 -> 27.4, 32 x 4096 x 11008
+//               28.3 -> 11.8; past one tile per CU, KS = 1: 300 x 4096 x 6000
+//               29.6 -> 21.7, 64 x 1024 x 32000 13.1 -> 9.7, 768 x 2048 x 5632
+//               24.1 -> 20.2 (128 x 128: 24.4).
+template <bool K4N>
+int launch_mid(const GemmArgs &args, int epi, uint32_t layout, hipStream_t stream) {
+    const long cus = compute_units();
+    auto tiles = [&](long bm, long bn) { return ((args.m + bm - 1) / bm) * ((args.n + bn - 1) / bn); };
+    const long t128 = tiles(128, 128), t12864 = tiles(128, 64), t64 = tiles(64, 64);
+    if (args.m > 64) {  // fewer rows would leave half of a 128-row tile empty
+        // (Short K over packed weights: their transposing LDS writes make the
+        // longer stage dearer, 2048 x 2048 x 5632 68.1 against 69.8 us.)
+        if (t128 > cus && !(args.k < 3072 && 4 * t128 <= 5 * cus))
+            return K4N && args.k < 3072 ? launch_gemm<128, 128, 64, 1, 1, K4N>(args, epi, layout, stream)
+                                        : launch_gemm<128, 128, 128, 2, 1, K4N>(args, epi, layout, stream);
+        if (t128 <= cus && 8 * t128 >= 5 * cus)
+            return launch_gemm<128, 128, 128, 2, 1, K4N, 2>(args, epi, layout, stream);
+        if (t12864 <= cus && 5 * t12864 >= 4 * cus)
+            return launch_gemm<128, 64, 128, 3, 1, K4N, 2>(args, epi, layout, stream);
+    }
+    if (t64 <= cus) return launch_gemm<64, 64, 128, 3, 1, K4N, 2>(args, epi, layout, stream);
+    return launch_gemm<64, 64, 128, 2, 1, K4N>(args, epi, layout, stream);
+}
+
 int run_gemm(const GemmArgs &args, int epi, uint32_t layout, hipStream_t stream) {
     if (gemv_path(args.m, args.k)) return dispatch_gemv<false>(args, FusedRows{}, epi, layout, stream);
     // 256 x 256 tiles once they give every CU a workgroup; 128 x 128 below that.
@@ -1230,20 +1311,11 @@ int run_gemm(const GemmArgs &args, int epi, uint32_t layout, hipStream_t stream)
         // (a timing-only copy) runs gate_up in 199 us and down in 152 us.
         return launch_stream(args, epi, stream);
     }
-    // Fewer 128 x 128 tiles than CUs (small M and N, e.g. one GPU's row shard
-    // of a down projection, M = 512, N = 4096, K = 14336): 64 x 64 tiles with
-    // 128-byte K stages fill the GPU instead (measured on MI355X: 115 -> 69 us
-    // for that shard; 31 -> 17 us at M = 256, K = N = 4096).
-    const long t128 = ((args.m + 127) / 128) * ((args.n + 127) / 128);
-    if (!big && t128 < cus) {
-        if (layout == QXT_W8A8_WEIGHT_K4N) return launch_gemm<64, 64, 128, 1, 1, true>(args, epi, layout, stream);
-        return launch_gemm<64, 64, 128, 1, 1, false>(args, epi, layout, stream);
-    }
-    if (layout == QXT_W8A8_WEIGHT_K4N)
-        return big ? launch_gemm<256, 256, 128, D, S, true>(args, epi, layout, stream)
-                   : launch_gemm<128, 128, 64, 1, 1, true>(args, epi, layout, stream);
-    return big ? launch_gemm<256, 256, 128, D, S, false>(args, epi, layout, stream)
-               : launch_gemm<128, 128, 64, 1, 1, false>(args, epi, layout, stream);
+    if (big)
+        return layout == QXT_W8A8_WEIGHT_K4N ? launch_gemm<256, 256, 128, D, S, true>(args, epi, layout, stream)
+                                             : launch_gemm<256, 256, 128, D, S, false>(args, epi, layout, stream);
+    return layout == QXT_W8A8_WEIGHT_K4N ? launch_mid<true>(args, epi, layout, stream)
+                                         : launch_mid<false>(args, epi, layout, stream);
 }
 
 int validate_gemm(const int8_t *a, size_t lda, const void *w, size_t ldw, uint32_t m, uint32_t n, uint32_t k,
