@@ -80,7 +80,7 @@ struct Q4ArgBatch {
     Q4Task task[kArgTasks];
 };
 
-// Two to fifteen rows on 16 x 16 matrix-core tiles (qxt_q4_0_rows.hip).  The
+// Two or more rows on 16 x 16 matrix-core tiles (qxt_q4_0_rows.hip).  The
 // single linear returns QXT_CAPABILITY_MISSING (no message, nothing launched)
 // for shapes it does not take.  The batch takes tasks of at most four rows each,
 // all native Q8_0 or (fp32_rows) all fp32, planned by q4_0_rows_plan (which

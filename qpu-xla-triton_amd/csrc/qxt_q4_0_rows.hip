@@ -1,5 +1,5 @@
-// Q4_0 x Q8_0 block-dot linear for two to fifteen rows on 16 x 16 matrix-core
-// tiles (gfx950), single linears and batches.
+// Q4_0 x Q8_0 block-dot linear for two or more rows on 16 x 16 matrix-core
+// tiles (gfx950): decode batches, short prompts, and batches of linears.
 //
 // Arithmetic as in qxt_q4_0.hip: per block an exact int32 dot, then
 // fl32(fl32(float(dot) * dw) * da), summed in block order.
@@ -554,17 +554,34 @@ static bool takes(const Q4Task &t, long tiles, long cus) {
     return !(blocks > 64 && blocks <= 128 && tiles > cus && 4 * tiles <= 5 * cus);
 }
 
+// Sixteen or more native rows: row groups of this kernel against the 64 x 64
+// prefill tiles (qxt_q4_0_tiled.hip), whose time is the K of one tile until
+// their grid fills the chip.  Both from sweeps on MI355X (us): this kernel 2.5 +
+// 3.6 ns per tile, group and 32 blocks (1.7 times that where one workgroup's LDS
+// takes a CU: more than 8 rows past K = 4096); the tiles 2.5 + 7.2 per 1024 of K,
+// from 300 workgroups 0.024 each.  Measured, tiles -> this kernel: 16 rows
+// 5632 x 2048 40.9 -> 7.2, 64 rows 41.3 -> 14.3, 128 rows 41.2 -> 34.2; 64 rows
+// 2048 x 5632 18.2 -> 12.6, 96 rows 18.1 -> 18.7 (not taken); 24 rows 4096 x 11008
+// 36.8 -> 24.9; 16 rows 2048 x 32000 24.0 -> 16.4, 24 rows 23.8 -> 31.2 (not taken).
+static bool takes_prefill(const Q4Task &t, long tiles) {
+    const int rpl = fits(t.blocks, 4) ? 4 : 2;
+    const double groups = (t.rows + 4 * rpl - 1) / (4 * rpl), chunks = (t.blocks + 31) / 32;
+    const double here = 2.5 + 3.6e-3 * (rpl == 4 && t.blocks > 128 ? 1.7 : 1.0) * tiles * groups * chunks;
+    const double workgroups = static_cast<double>((t.rows + 63) / 64) * ((t.ncols + 63) / 64);
+    return 1.1 * here < 2.5 + t.blocks / 32.0 * std::max(7.2, 0.024 * workgroups);
+}
+
 int q4_0_rows_linear(const Q4Task &t, hipStream_t stream) {
-    if (t.rows < 2 || t.rows > 15 || !layout_ok(t)) return QXT_CAPABILITY_MISSING;
+    if (t.rows < 2 || !layout_ok(t)) return QXT_CAPABILITY_MISSING;
     const long tiles = (t.ncols + 15) / 16, cus = compute_units();
-    if (!takes(t, tiles, cus)) return QXT_CAPABILITY_MISSING;
+    if (t.rows > 15 ? !takes_prefill(t, tiles) : !takes(t, tiles, cus)) return QXT_CAPABILITY_MISSING;
     // The fewest rows per lane that leave every workgroup a CU of its own;
     // larger grids take all rows at once (K = 5632, N = 2048, 5 rows: two row
     // groups 6.4 us, one 7.0; K = 2048, N = 5632: 6.6 and 5.3).
     int rpl = 0;
     for (int r = 1; r <= 4 && rpl == 0; ++r)
         if (fits(t.blocks, r) && (tiles * ((t.rows + 4 * r - 1) / (4 * r)) <= cus || 4 * r >= t.rows)) rpl = r;
-    if (rpl == 0) rpl = fits(t.blocks, 2) ? 2 : 1;
+    if (rpl == 0) rpl = fits(t.blocks, 4) ? 4 : fits(t.blocks, 2) ? 2 : 1;
     if (!fits(t.blocks, rpl)) return QXT_CAPABILITY_MISSING;
     const long groups = (t.rows + 4 * rpl - 1) / (4 * rpl);
     // Half-unit chunks while the grid is latency-bound: half the instructions

@@ -161,3 +161,18 @@ def test_row_tile_batch_captured_and_replayed_reads_the_rows_of_each_replay() ->
             torch.cuda.synchronize()
             np.testing.assert_array_equal(
                 out.cpu().numpy(), oracle.q4_0_q8_0_reference(oracle.quantize_q8_0_blocks(rows), wt))
+
+
+@pytest.mark.parametrize("rows,blocks,n,wcol0,ncols", [
+    (16, 64, 70, 0, 70),       # a whole group of sixteen rows, or several smaller ones
+    (17, 24, 300, 5, 290),     # one row past a group
+    (33, 40, 4200, 0, 4200),   # groups of sixteen rows over more tiles than CUs
+    (100, 128, 256, 0, 256),
+    (40, 176, 2048, 0, 2048),  # past K = 4096: one workgroup's LDS a CU
+    (24, 344, 4100, 0, 4100),  # groups of eight rows (LDS)
+    (300, 64, 100, 0, 100),
+    (64, 64, 5632, 0, 5632),   # the last row count here, the prefill tiles past it
+    (96, 64, 5632, 0, 5632),
+])
+def test_short_prompts_on_row_tiles_bit_exact(rows: int, blocks: int, n: int, wcol0: int, ncols: int) -> None:
+    _check_linear("native", rows, blocks, n, wcol0, ncols)
