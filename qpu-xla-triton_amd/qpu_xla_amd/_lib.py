@@ -226,6 +226,8 @@ _lib: ctypes.CDLL | None = None
 def load() -> ctypes.CDLL:
     """Load (once) and return the library with typed signatures."""
     global _lib
+    if _lib is not None:
+        return _lib
     with _lock:
         if _lib is not None:
             return _lib
@@ -263,7 +265,9 @@ def check(status: int) -> None:
 
 def call(name: str, *args: Any) -> None:
     """Call an entry point and raise on a non-OK status."""
-    check(getattr(load(), name)(*args))
+    status = getattr(_lib or load(), name)(*args)
+    if status != OK:
+        check(status)
 
 
 def set_failure_mask(mask: int) -> None:

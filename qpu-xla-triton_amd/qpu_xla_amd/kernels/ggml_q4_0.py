@@ -20,7 +20,7 @@ from typing import Any
 import torch
 
 from qpu_xla_amd import _lib
-from qpu_xla_amd._tensors import PACKED_WORD_DTYPES, ptr, require_gpu, row_stride, rows_are_dense, stream_handle
+from qpu_xla_amd._tensors import PACKED_WORD_DTYPES, on_gpu, ptr, require_gpu, row_stride, rows_are_dense, stream_handle
 from qpu_xla_amd.errors import KernelError
 from qpu_xla_amd.kernel import Kernel
 
@@ -342,9 +342,10 @@ def supports_ggml_q4_0_q8_0_tiled_linear(
 ) -> bool:
     """Whether split tensors meet the tiled contract (ggml_q4_0.py:886-920), widened to any M and N."""
     tensors = (activation_q, activation_scales, weight_q, weight_scales, destination)
-    if not all(isinstance(t, torch.Tensor) and t.dim() == 2 for t in tensors):
-        return False
-    if any(t.device.type != "cuda" for t in tensors) or len({t.device for t in tensors}) != 1:
+    for t in tensors:
+        if not isinstance(t, torch.Tensor) or t.dim() != 2 or not t.is_contiguous():
+            return False
+    if not on_gpu(*tensors):
         return False
     if activation_q.dtype not in (torch.uint8, torch.int8) or weight_q.dtype not in PACKED_WORD_DTYPES:
         return False
@@ -357,14 +358,13 @@ def supports_ggml_q4_0_q8_0_tiled_linear(
         return False
     blocks = columns // Q4_0_BLOCK_ELEMENTS
     outputs = weight_q.shape[1]
-    shapes_ok = (
+    return (
         outputs > 0
-        and tuple(activation_scales.shape) == (rows, blocks)
-        and tuple(weight_q.shape) == (blocks * 8, outputs)
-        and tuple(weight_scales.shape) == (blocks, outputs)
-        and tuple(destination.shape) == (rows, outputs)
+        and activation_scales.shape == (rows, blocks)
+        and weight_q.shape == (blocks * 8, outputs)
+        and weight_scales.shape == (blocks, outputs)
+        and destination.shape == (rows, outputs)
     )
-    return shapes_ok and all(t.is_contiguous() for t in tensors)
 
 
 def tiled_grid(rows: int, outputs: int) -> tuple[int, int, int]:

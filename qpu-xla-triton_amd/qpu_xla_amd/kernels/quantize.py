@@ -37,7 +37,7 @@ def quantize_q8_0(x: torch.Tensor, out: torch.Tensor | None = None, *, stream: A
         raise ValueError("quantize_q8_0: K must be a multiple of 32")
     if out is None:
         out = torch.empty((rows, columns // QK, Q8_0_BLOCK_BYTES), dtype=torch.uint8, device=x.device)
-    elif out.dtype != torch.uint8 or tuple(out.shape) != (rows, columns // QK, Q8_0_BLOCK_BYTES) or not out[0].is_contiguous():
+    elif out.dtype != torch.uint8 or tuple(out.shape) != (rows, columns // QK, Q8_0_BLOCK_BYTES) or not rows_are_dense(out):
         raise ValueError("quantize_q8_0: out must be uint8 [M, K/32, 34] with contiguous rows")
     require_gpu("quantize_q8_0", x, out)
     _lib.call("qxt_quantize_q8_0", ptr(x), row_stride(x), ptr(out), row_stride(out), rows, columns, stream_handle(stream))
@@ -85,7 +85,7 @@ def quantize_q4_0(w: torch.Tensor, out: torch.Tensor | None = None, *, stream: A
         raise ValueError("quantize_q4_0: K must be a multiple of 32")
     if out is None:
         out = torch.empty((rows, columns // QK, Q4_0_BLOCK_BYTES), dtype=torch.uint8, device=w.device)
-    elif out.dtype != torch.uint8 or tuple(out.shape) != (rows, columns // QK, Q4_0_BLOCK_BYTES) or not out[0].is_contiguous():
+    elif out.dtype != torch.uint8 or tuple(out.shape) != (rows, columns // QK, Q4_0_BLOCK_BYTES) or not rows_are_dense(out):
         raise ValueError("quantize_q4_0: out must be uint8 [N, K/32, 18] with contiguous rows")
     require_gpu("quantize_q4_0", w, out)
     _lib.call("qxt_quantize_q4_0", ptr(w), row_stride(w), ptr(out), row_stride(out), rows, columns, stream_handle(stream))
