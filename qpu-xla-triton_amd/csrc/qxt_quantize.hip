@@ -27,6 +27,7 @@ namespace qxt {
 namespace {
 
 constexpr int kThreads = 256;
+constexpr int kWideThreads = 1024;  // of a workgroup per row, few long rows
 
 __device__ __forceinline__ float group8_max(float v) {
     v = fmaxf(v, __shfl_xor(v, 1, 8));
@@ -245,25 +246,26 @@ __global__ __launch_bounds__(kBandThreads) void geglu_q8_0_band_kernel(
 
 // ------------------------------------------------------------- per-row int8
 
+template <int NT>
 __device__ __forceinline__ float block_max(float v, float *scratch) {
     for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
     const int wave = threadIdx.x >> 6;
     if ((threadIdx.x & 63) == 0) scratch[wave] = v;
     __syncthreads();
     v = scratch[0];
-    for (int w = 1; w < kThreads / 64; ++w) v = fmaxf(v, scratch[w]);
+    for (int w = 1; w < NT / 64; ++w) v = fmaxf(v, scratch[w]);
     return v;
 }
 
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 
-// NV > 0: the row (columns % 4 == 0, <= 1024 * NV columns) is held in registers.
-template <int NV, bool VEC>
-__global__ __launch_bounds__(kThreads) void rows_int8_kernel(const float *__restrict__ x, size_t x_stride,
+// The row (columns % 4 == 0, <= 4 * NT * NV columns) is held in registers.
+template <int NV, bool VEC, int NT>
+__global__ __launch_bounds__(NT) void rows_int8_kernel(const float *__restrict__ x, size_t x_stride,
                                                              int8_t *__restrict__ q, size_t q_stride,
                                                              float *__restrict__ scales, uint32_t columns,
                                                              uint32_t padded, bool floor) {
-    __shared__ float scratch[kThreads / 64];
+    __shared__ float scratch[NT / 64];
     const uint32_t row = blockIdx.x;
     const float *src = reinterpret_cast<const float *>(reinterpret_cast<const uint8_t *>(x) + row * x_stride);
     int8_t *dst = q + row * q_stride;
@@ -278,7 +280,7 @@ __global__ __launch_bounds__(kThreads) void rows_int8_kernel(const float *__rest
         // against loads guarded per lane.
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
-            const uint32_t c = min(threadIdx.x + i * kThreads, chunks - 1);
+            const uint32_t c = min(threadIdx.x + i * NT, chunks - 1);
             const v4u raw = __builtin_nontemporal_load(reinterpret_cast<const v4u *>(src) + c);
             v[i] = make_float4(__uint_as_float(raw[0]), __uint_as_float(raw[1]), __uint_as_float(raw[2]),
                                __uint_as_float(raw[3]));
@@ -289,14 +291,14 @@ __global__ __launch_bounds__(kThreads) void rows_int8_kernel(const float *__rest
     } else {
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
-            const uint32_t c = threadIdx.x + i * kThreads;
+            const uint32_t c = threadIdx.x + i * NT;
             if (c < chunks) {
                 v[i] = load4<VEC>(src + 4 * c);
                 amax = fmaxf(amax, fmaxf(fmaxf(fabsf(v[i].x), fabsf(v[i].y)), fmaxf(fabsf(v[i].z), fabsf(v[i].w))));
             }
         }
     }
-    const float s = row_scale(block_max(amax, scratch), floor);
+    const float s = row_scale(block_max<NT>(amax, scratch), floor);
     // Every row scale of the 1/127 floor takes the reciprocal form (measured
     // on MI355X at 4096 rows: K = 14336 50.8 -> 47.0 us, K = 4096 15.6 ->
     // 14.4 us against a division per element).
@@ -308,7 +310,7 @@ __global__ __launch_bounds__(kThreads) void rows_int8_kernel(const float *__rest
         auto quant = [&](float x) { return recip ? quant_recip(x, s, r) : quant_div(x, s); };
 #pragma unroll
         for (int i = 0; i < NV; ++i) {
-            const uint32_t c = threadIdx.x + i * kThreads;
+            const uint32_t c = threadIdx.x + i * NT;
             if (c < chunks) {
                 const uint32_t word = pack_bytes(quant(v[i].x), quant(v[i].y), quant(v[i].z), quant(v[i].w));
                 if constexpr (VEC) {
@@ -323,7 +325,7 @@ __global__ __launch_bounds__(kThreads) void rows_int8_kernel(const float *__rest
         quantise(std::true_type{});
     else
         quantise(std::false_type{});
-    for (uint32_t c = columns + threadIdx.x; c < padded; c += kThreads) dst[c] = 0;
+    for (uint32_t c = columns + threadIdx.x; c < padded; c += NT) dst[c] = 0;
     if (threadIdx.x == 0) scales[row] = s;
 }
 
@@ -338,7 +340,7 @@ __global__ __launch_bounds__(kThreads) void rows_int8_generic_kernel(const float
     int8_t *dst = q + row * q_stride;
     float amax = 0.0f;
     for (uint32_t c = threadIdx.x; c < columns; c += kThreads) amax = fmaxf(amax, fabsf(src[c]));
-    const float s = row_scale(block_max(amax, scratch), floor);
+    const float s = row_scale(block_max<kThreads>(amax, scratch), floor);
     for (uint32_t c = threadIdx.x; c < columns; c += kThreads) dst[c] = static_cast<int8_t>(quant_div(src[c], s));
     for (uint32_t c = columns + threadIdx.x; c < padded; c += kThreads) dst[c] = 0;
     if (threadIdx.x == 0) scales[row] = s;
@@ -510,14 +512,27 @@ int qxt_quantize_rows_int8(const float *x, size_t x_row_stride, int8_t *q, size_
     const bool floor = (flags & QXT_QUANT_NO_SCALE_FLOOR) == 0;
     const bool vec = columns % 4 == 0 && aligned(x, 16) && x_row_stride % 16 == 0 && aligned(q, 4) &&
                      q_row_stride % 4 == 0;
-    const uint32_t per_thread = (columns / 4 + kThreads - 1) / kThreads;
+    const uint32_t chunks = columns / 4;
     auto kernel = rows_int8_generic_kernel;
-    if (vec && per_thread <= 1) kernel = rows_int8_kernel<1, true>;
-    else if (vec && per_thread <= 2) kernel = rows_int8_kernel<2, true>;
-    else if (vec && per_thread <= 4) kernel = rows_int8_kernel<4, true>;
-    else if (vec && per_thread <= 8) kernel = rows_int8_kernel<8, true>;
-    else if (vec && per_thread <= 16) kernel = rows_int8_kernel<16, true>;
-    return launch("rows_int8_kernel", kernel, dim3(rows), dim3(kThreads), 0, as_stream(stream), x, x_row_stride, q,
+    uint32_t threads = kThreads;
+    // While a CU holds at most two rows, their time is one thread's chain of
+    // conversions, so rows longer than 4096 take 1024 threads.  Measured on
+    // MI355X, 256 -> 1024 threads (us, rotated inputs): 48 rows, K = 5632 3.44 ->
+    // 3.06, 11008 4.73 -> 3.79, 14336 5.16 -> 4.05; 512 rows 5.23 -> 5.17, 8.23 ->
+    // 7.38, 9.57 -> 8.74.  Not past the line: 1024 rows, K = 5632 7.35 -> 8.27,
+    // 14336 15.14 -> 15.32; K = 4096, 48 rows 3.13 -> 3.05 but 512 rows 4.21 -> 4.54.
+    if (vec && chunks > 1024 && chunks <= 4096 && rows <= 2u * static_cast<uint32_t>(compute_units())) {
+        threads = kWideThreads;
+        kernel = chunks <= 2048 ? rows_int8_kernel<2, true, kWideThreads> : rows_int8_kernel<4, true, kWideThreads>;
+    } else if (vec) {
+        const uint32_t per_thread = (chunks + kThreads - 1) / kThreads;
+        if (per_thread <= 1) kernel = rows_int8_kernel<1, true, kThreads>;
+        else if (per_thread <= 2) kernel = rows_int8_kernel<2, true, kThreads>;
+        else if (per_thread <= 4) kernel = rows_int8_kernel<4, true, kThreads>;
+        else if (per_thread <= 8) kernel = rows_int8_kernel<8, true, kThreads>;
+        else if (per_thread <= 16) kernel = rows_int8_kernel<16, true, kThreads>;
+    }
+    return launch("rows_int8_kernel", kernel, dim3(rows), dim3(threads), 0, as_stream(stream), x, x_row_stride, q,
                   q_row_stride, scales, columns, padded_columns, floor);
 }
 
