@@ -65,23 +65,28 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_rsrc(const void *base, 
 
 constexpr uint32_t kOutOfRange = 0x80000000u;  // operands are < 2 GiB, so this offset is always out of range
 
-// Global -> register staging of one K stage (BKT bytes of K): A rows [m0, m0+BM)
+// Waves of a group of w8a8_gemm_kernel along each side of its tile.
+constexpr int waves_along(int side) { return side >= 64 ? 2 : 1; }
+
+// Global -> register staging of one K stage (BKT bytes of K) by one group of
+// waves: A rows [m0, m0+BM)
 // and B columns [n0, n0+BN) as 16-byte chunks, zeros outside the matrices.
 template <int BM, int BN, int BKT, bool K4N>
 struct StageRegs {
+    static constexpr int kGroup = 64 * waves_along(BM) * waves_along(BN);  // threads
     static constexpr int CPR = BKT / 16;  // chunks per LDS row
-    static constexpr int A_CHUNKS = BM * CPR / kThreads;
-    static constexpr int B_CHUNKS = BN * CPR / kThreads;
+    static constexpr int A_CHUNKS = BM * CPR / kGroup;
+    static constexpr int B_CHUNKS = BN * CPR / kGroup;
     static constexpr int STORES = A_CHUNKS + (K4N ? 4 : 1) * B_CHUNKS;  // LDS write instructions
     v4u a[A_CHUNKS];
     v4u b[B_CHUNKS];
 
     __device__ __forceinline__ void load(const GemmArgs &args, __amdgpu_buffer_rsrc_t ra, __amdgpu_buffer_rsrc_t rb,
                                          int m0, int n0, int k0) {
-        const int tid = threadIdx.x % kThreads;
+        const int tid = threadIdx.x % kGroup;
 #pragma unroll
         for (int i = 0; i < A_CHUNKS; ++i) {
-            const int c = tid + i * kThreads;
+            const int c = tid + i * kGroup;
             const int row = c / CPR, kc = c % CPR;
             const int gm = m0 + row, gk = k0 + kc * 16;
             const uint32_t off = (gm < args.m && gk < args.k) ? static_cast<uint32_t>(gm) * args.lda + gk : kOutOfRange;
@@ -89,7 +94,7 @@ struct StageRegs {
         }
 #pragma unroll
         for (int i = 0; i < B_CHUNKS; ++i) {
-            const int c = tid + i * kThreads;
+            const int c = tid + i * kGroup;
             uint32_t off;
             if constexpr (!K4N) {
                 const int row = c / CPR, kc = c % CPR;
@@ -106,16 +111,16 @@ struct StageRegs {
     }
 
     __device__ __forceinline__ void store(uint8_t *As, uint8_t *Bs) const {
-        const int tid = threadIdx.x % kThreads;
+        const int tid = threadIdx.x % kGroup;
         constexpr int ROW = BKT + 16;
 #pragma unroll
         for (int i = 0; i < A_CHUNKS; ++i) {
-            const int c = tid + i * kThreads;
+            const int c = tid + i * kGroup;
             *reinterpret_cast<v4u *>(As + (c / CPR) * ROW + (c % CPR) * 16) = a[i];
         }
 #pragma unroll
         for (int i = 0; i < B_CHUNKS; ++i) {
-            const int c = tid + i * kThreads;
+            const int c = tid + i * kGroup;
             if constexpr (!K4N) {
                 *reinterpret_cast<v4u *>(Bs + (c / CPR) * ROW + (c % CPR) * 16) = b[i];
             } else {
@@ -294,19 +299,20 @@ __device__ __forceinline__ void store_tile_rows(const GemmArgs &args, const v16i
 // the staged scales behind it.
 constexpr int kEpilogueLds = 128 * 1024 + 3 * 256 * 4;
 
-// BM x BN output tile per 256-thread workgroup; waves 2 x 2, each (BM/2) x (BN/2)
-// as (BM/64) x (BN/64) blocks of 32 x 32.  K advances BKT bytes per stage
-// through two LDS buffers (rows padded by 16 bytes, so the 16-byte fragment
+// BM x BN output tile per group of waves, 2 x 2 of them, each (BM/2) x (BN/2) as
+// (BM/64) x (BN/64) blocks of 32 x 32 (one wave along a side of 32).  K advances
+// BKT bytes per stage through two LDS buffers (rows padded by 16 bytes, so the 16-byte fragment
 // reads of 8 consecutive rows hit distinct banks): the next stage's global
 // loads are issued before the current stage's MFMAs and written to the other
 // buffer after them, one barrier per stage.  Within a stage the fragments of
 // the next 32-deep k step are read from LDS while the current step's MFMAs run.
 //
-// KS > 1: KS groups of four waves share the tile, group g taking K stages g,
+// KS > 1: KS groups of waves share the tile, group g taking K stages g,
 // g + KS, ... with buffers of its own; the groups' exact int32 sums are added
 // through LDS at the end.
 template <int BM, int BN, int BKT, int DEPTH, int STORE_KS, int KS, bool K4N, int EPI>
-__global__ __launch_bounds__(KS * kThreads) void w8a8_gemm_kernel(GemmArgs args) {
+__global__ __launch_bounds__(KS * 64 * waves_along(BM) * waves_along(BN)) void w8a8_gemm_kernel(GemmArgs args) {
+    constexpr int WY = waves_along(BM), WX = waves_along(BN);
     constexpr int ROW = BKT + 16;
     constexpr int STAGE = (BM + BN) * ROW;
     constexpr int KSTEPS = BKT / 32;
@@ -315,14 +321,14 @@ __global__ __launch_bounds__(KS * kThreads) void w8a8_gemm_kernel(GemmArgs args)
     static_assert(STORE_KS >= 0 && STORE_KS < KSTEPS, "store step inside the stage");
     static_assert((KS - 1) * BM * BN * 4 + 3 * 256 * 4 <= KS * 2 * STAGE, "the partial sums reuse the operand buffers");
     __shared__ __attribute__((aligned(16))) uint8_t shared[KS * 2 * STAGE];
-    const int group = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kThreads));
+    const int group = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / (64 * WY * WX)));
     uint8_t *const smem = shared + group * 2 * STAGE;
 
-    constexpr int WM = BM / 2, WN = BN / 2;    // per-wave sub-tile
+    constexpr int WM = BM / WY, WN = BN / WX;  // per-wave sub-tile
     constexpr int TM = WM / 32, TN = WN / 32;  // 32x32 blocks per wave
     const int lane = threadIdx.x & 63;
-    const int wave = (threadIdx.x >> 6) & 3;
-    const int wm = wave >> 1, wn = wave & 1;
+    const int wave = (threadIdx.x >> 6) % (WY * WX);
+    const int wm = wave / WX, wn = wave % WX;
     const int m0 = blockIdx.y * BM;
     const int n0 = blockIdx.x * BN;
     const __amdgpu_buffer_rsrc_t ra = buffer_rsrc(args.a, args.a_bytes);
@@ -412,7 +418,7 @@ __global__ __launch_bounds__(KS * kThreads) void w8a8_gemm_kernel(GemmArgs args)
         // 16-byte piece per lane and register quad.
         v4i *parts = reinterpret_cast<v4i *>(shared + 3 * 256 * 4);
         auto piece = [&](int g, int i, int j, int q) -> v4i & {
-            return parts[(((((g - 1) * 4 + wave) * TM + i) * TN + j) * 4 + q) * 64 + lane];
+            return parts[(((((g - 1) * WY * WX + wave) * TM + i) * TN + j) * 4 + q) * 64 + lane];
         };
         if (group > 0) {
 #pragma unroll
@@ -1074,7 +1080,8 @@ int launch_gemm(GemmArgs args, int epi, uint32_t layout, hipStream_t stream) {
     auto kernel = epi == EPI_I32        ? w8a8_gemm_kernel<BM, BN, BKT, DEPTH, STORE_KS, KS, K4N, EPI_I32>
                   : epi == EPI_DEQUANT ? w8a8_gemm_kernel<BM, BN, BKT, DEPTH, STORE_KS, KS, K4N, EPI_DEQUANT>
                                        : w8a8_gemm_kernel<BM, BN, BKT, DEPTH, STORE_KS, KS, K4N, EPI_DEQUANT_BIAS>;
-    return launch("w8a8_gemm_kernel", kernel, grid, dim3(KS * kThreads), 0, stream, args);
+    return launch("w8a8_gemm_kernel", kernel, grid, dim3(KS * 64 * waves_along(BM) * waves_along(BN)), 0,
+                  stream, args);
 }
 
 int launch_stream(const GemmArgs &args, int epi, hipStream_t stream) {
@@ -1269,6 +1276,14 @@ bool gemv_path(int m, int k) {
 //               28.3 -> 11.8; past one tile per CU, KS = 1: 300 x 4096 x 6000
 //               29.6 -> 21.7, 64 x 1024 x 32000 13.1 -> 9.7, 768 x 2048 x 5632
 //               24.1 -> 20.2 (128 x 128: 24.4).
+// While even 32 x 32 tiles, or 64 x 32, leave at most one to a CU they take the
+// call from K = 1024: a CU takes in half of the columns or less, and eight or
+// four groups of waves (KS) keep as many loads in flight.  64 x 64 -> 32 x 32:
+// 8 x 14336 x 4096 27.9 -> 21.0, 48 x 14336 x 4096 33.4 -> 22.5, 16 x 14336 x 512
+// 26.7 -> 16.1, 8 x 4096 x 4096 10.4 -> 8.6, packed 8 x 14336 x 4096 48.0 -> 22.2; 512 of
+// K 3.8 -> 4.6, a second round of tiles (8 x 4096 x 8800) 13.0 -> 16.7, not taken.
+// 64 x 64 -> 64 x 32: 128 x 14336 x 4096 35.4 -> 27.8, 200 x 4096 x 2048 10.5 -> 8.9,
+// 40 x 8192 x 8192 24.1 -> 19.2; a second round (64 x 4096 x 11008) 16.4 -> 20.7.
 template <bool K4N>
 int launch_mid(const GemmArgs &args, int epi, uint32_t layout, hipStream_t stream) {
     const long cus = compute_units();
@@ -1285,6 +1300,10 @@ int launch_mid(const GemmArgs &args, int epi, uint32_t layout, hipStream_t strea
         if (t12864 <= cus && 5 * t12864 >= 4 * cus)
             return launch_gemm<128, 64, 128, 3, 1, K4N, 2>(args, epi, layout, stream);
     }
+    if (args.k >= 1024 && tiles(32, 32) <= cus)
+        return launch_gemm<32, 32, 128, 3, 1, K4N, 8>(args, epi, layout, stream);
+    if (args.k >= 1024 && tiles(64, 32) <= cus)
+        return launch_gemm<64, 32, 128, 3, 1, K4N, 4>(args, epi, layout, stream);
     if (t64 <= cus) return launch_gemm<64, 64, 128, 3, 1, K4N, 2>(args, epi, layout, stream);
     return launch_gemm<64, 64, 128, 2, 1, K4N>(args, epi, layout, stream);
 }
