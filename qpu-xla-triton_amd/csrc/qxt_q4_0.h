@@ -3,6 +3,7 @@
 #pragma once
 
 #include "qxt_common.h"
+#include "qxt_q4_0_rows_plan.h"
 
 namespace qxt {
 
@@ -84,12 +85,12 @@ struct Q4ArgBatch {
 // single linear returns QXT_CAPABILITY_MISSING (no message, nothing launched)
 // for shapes it does not take.  The batch takes tasks of at most four rows each,
 // all native Q8_0 or (fp32_rows) all fp32, planned by q4_0_rows_plan (which
-// sets every task's cpw and returns the threads of a workgroup); `args` or,
-// when that is null, the device tables `tasks` and `items`.
+// sets every task's cpw); `args` or, when that is null, the device tables
+// `tasks` and `items`.
 int q4_0_rows_linear(const Q4Task &t, hipStream_t stream);
-bool q4_0_rows_batch_supported(const Q4Task &t);
-int q4_0_rows_plan(Q4Task *tasks, uint32_t count, size_t *lds);
-int q4_0_rows_batch(const Q4ArgBatch *args, const Q4Task *tasks, const Q4Item *items, uint32_t grid, int threads,
-                    size_t lds, int layout, bool fp32_rows, hipStream_t stream);
+bool q4_0_rows_batch_takes(const Q4Task *tasks, uint32_t count);
+RowsPlan q4_0_rows_plan(Q4Task *tasks, uint32_t count);
+int q4_0_rows_batch(const Q4ArgBatch *args, const Q4Task *tasks, const Q4Item *items, uint32_t grid,
+                    const RowsPlan &plan, int layout, bool fp32_rows, hipStream_t stream);
 
 }  // namespace qxt

@@ -1448,7 +1448,8 @@ struct qxt_q4_0_batch {
     int split = 1;     // waves per unit (one-row prefetch batches of narrow items)
     int threads = kThreads;  // 256, or 512 / 1024 for split prefetch batches
     size_t lds = 0;
-    bool rows = false;     // the row-tile kernels (tasks of two to four rows)
+    bool rows = false;     // the row-tile kernels (tasks of two to four rows), by rows_plan
+    RowsPlan rows_plan{};
     bool rows_fp32 = false;  // they quantise fp32 rows themselves
     bool in_args = false;  // tasks and items travel in the kernel arguments
     Q4ArgBatch args{};
@@ -1762,14 +1763,22 @@ int qxt_q4_0_batch_prepare(const qxt_q4_0_task *tasks, uint32_t count, qxt_q4_0_
     // its weights and quantises it while they are in flight.  A batch whose
     // tiles were narrowed (too few columns to fill the chip) runs it with
     // kPrefetchUnits units per thread, its tiles planned for that.
-    // Batches with tasks of two to four rows run the row-tile kernels, which
-    // quantise fp32 rows themselves when every task of a small batch gives
-    // them and read the pre-pass's Q8_0 rows otherwise.
-    bool row_tiles = mr != 1;
-    for (uint32_t i = 0; i < count && row_tiles; ++i) {
-        Q4Task t = host[i];
-        t.x = nullptr;
-        row_tiles = q4_0_rows_batch_supported(t);
+    // Batches with tasks of two to four rows mostly run the row-tile kernels,
+    // which quantise fp32 rows themselves when every task of a small batch
+    // gives them and read the pre-pass's Q8_0 rows otherwise.
+    const bool row_tiles = mr != 1 && q4_0_rows_batch_takes(host.data(), count);
+    if (row_tiles) {
+        // Long K first: a last round of workgroups that each take several
+        // passes over K leaves the chip idle behind it (whole steps of 28
+        // shapes, MI355X: 7 % of the time in the geometric mean).
+        std::vector<uint32_t> order(count), place(count);
+        for (uint32_t i = 0; i < count; ++i) order[i] = i;
+        std::stable_sort(order.begin(), order.end(),
+                         [&](uint32_t a, uint32_t b) { return host[a].blocks > host[b].blocks; });
+        std::vector<Q4Task> sorted(count);
+        for (uint32_t i = 0; i < count; ++i) sorted[i] = host[order[i]], place[order[i]] = i;
+        host.swap(sorted);
+        for (uint32_t &i : job_task) i = place[i];
     }
     bool prefetch_candidate = mr == 1;
     for (uint32_t i = 0; i < count && prefetch_candidate; ++i) prefetch_candidate = prefetch_chunks(host[i]) > 0;
@@ -1821,9 +1830,9 @@ int qxt_q4_0_batch_prepare(const qxt_q4_0_task *tasks, uint32_t count, qxt_q4_0_
     }
     size_t lds = 0;
     std::vector<Q4Item> items;
-    int threads = kThreads;
+    RowsPlan rows_plan{};
     if (row_tiles) {
-        threads = q4_0_rows_plan(host.data(), count, &lds);
+        rows_plan = q4_0_rows_plan(host.data(), count);
         for (uint32_t i = 0; i < count; ++i)
             for (int c = 0; c < host[i].ncols; c += host[i].cpw)
                 items.push_back({static_cast<int>(i), c, std::min(host[i].cpw, host[i].ncols - c)});
@@ -1893,7 +1902,7 @@ int qxt_q4_0_batch_prepare(const qxt_q4_0_task *tasks, uint32_t count, qxt_q4_0_
     batch->mr = mr;
     batch->rows = row_tiles;
     batch->rows_fp32 = rows_fp32;
-    batch->threads = threads;
+    batch->rows_plan = rows_plan;
     batch->layout = layout;
     // The prefetch kernel runs exactly the batches planned for it.
     batch->prefetch = 0;
@@ -1958,7 +1967,7 @@ int qxt_q4_0_batch_launch(const qxt_q4_0_batch *batch, void *stream) {
     }
     if (batch->rows)
         return q4_0_rows_batch(batch->in_args ? &batch->args : nullptr, batch->tasks, batch->items, batch->grid,
-                               batch->threads, batch->lds, batch->layout, batch->rows_fp32, as_stream(stream));
+                               batch->rows_plan, batch->layout, batch->rows_fp32, as_stream(stream));
     const BatchKernel kernel =
         batch_kernel(batch->mr, batch->layout, batch->prefetch, batch->upt, batch->split, batch->threads);
     const dim3 block(batch->threads);

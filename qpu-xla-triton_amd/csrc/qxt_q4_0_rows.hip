@@ -25,7 +25,9 @@
 // terms in registers; then the waves add them in turn to the tile's running
 // sums (LDS), which keeps the block order.  A workgroup walks several column
 // tiles where the grid is large, the next tile's weights in flight while a
-// tile is computed; its activation rows are staged in LDS once.
+// tile is computed; its activation rows are staged in LDS once.  In a batch
+// whose longest K asks for more waves than a task has chunks, the task's
+// workgroups compute waves / chunks column tiles side by side.
 //
 // What bounds it: small grids, the instructions of one wave (about 450 per
 // chunk of 32 blocks at one row per lane, 6 to 7 cycles each with one wave per
@@ -33,7 +35,7 @@
 // Measured on MI355X against the kernels it replaces (bit-identical): single
 // linears in takes() below; a staged decode step of four rows over Llama-7B
 // class layers (K = 4096 / 11008, 16 stages) 557 -> 239 us; whole-step batches of
-// four rows 382 -> 134 us (the same four layers, two launches) and 196 -> 149 us
+// four rows 387 -> 122 us (the same four layers, two launches) and 196 -> 139 us
 // (154 TinyLlama linears).
 #include <algorithm>
 #include <type_traits>
@@ -47,7 +49,6 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef unsigned int v2u __attribute__((ext_vector_type(2)));
 
 constexpr int kMaxPasses = 4;    // chunks per wave and tile
-constexpr size_t kLds = 160 * 1024;
 
 // Most waves of a workgroup, by what a lane holds (registers).
 template <int NB>
@@ -313,7 +314,10 @@ __device__ __forceinline__ void chunk_terms(const uint32_t (&w)[36], const uint8
 
 // Rows [r0, r0 + m) of columns [col_base, col_base + ncols) of one linear.
 // X: the activation is fp32 rows (RPL = 1, NB = 8), else native Q8_0 rows.
-template <int RPL, int LAYOUT, int NB, bool X = false>
+// GROUPS: the workgroup may have more waves than K has chunks; each `chunks`
+// of them are a group with a column tile of its own (waves past the last group
+// only run the barriers).
+template <int RPL, int LAYOUT, int NB, bool X = false, bool GROUPS = false>
 __device__ __forceinline__ void rows_item(const Q4Task &t, int r0, int col_base, int ncols) {
     using G = RowsGeo<RPL, NB>;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -324,10 +328,15 @@ __device__ __forceinline__ void rows_item(const Q4Task &t, int r0, int col_base,
     const int chunks = (units + G::kUnits - 1) / G::kUnits;
     const int half = (lane >> 4) & 1;
     const int passes = (chunks + waves - 1) / waves;
+    const int groups = GROUPS ? max(1, waves / chunks) : 1;
+    const int span = GROUPS ? min(waves, chunks) : waves;  // waves of a group
+    const int group = GROUPS ? wave / span : 0;
+    const int gwave = GROUPS ? wave - group * span : wave;  // this wave in its group
     const int m = min(t.rows - r0, G::kRows);
-    float *run = reinterpret_cast<float *>(lds + static_cast<size_t>(chunks) * G::kChunkBytes);
+    float *run = reinterpret_cast<float *>(lds + static_cast<size_t>(chunks) * G::kChunkBytes) +
+                 (GROUPS ? min(group, groups - 1) * (RPL * 64) : 0);
 
-    // This wave's chunks are wave, wave + waves, ...; the first one's rows are
+    // This wave stages chunks wave, wave + waves, ...; the first one's rows are
     // requested last, before the first tile's weights, and staged while those
     // are in flight.
     std::conditional_t<X, RowRegs, PairRegs<RPL, NB>> a;
@@ -349,32 +358,33 @@ __device__ __forceinline__ void rows_item(const Q4Task &t, int r0, int col_base,
     request(min(wave, chunks - 1));
     __builtin_amdgcn_sched_barrier(0);
     const int tiles = (ncols + 15) >> 4;
-    const int steps = tiles * passes;
-    // Step q: column tile q / passes, chunk (q % passes) * waves + wave.
-    int tile = 0, pass = 0;
+    const int steps = (tiles + groups - 1) / groups * passes;
+    // Step q: column tile groups * (q / passes) + group, chunk (q % passes) *
+    // span + gwave.
+    int tile = group, pass = 0;
     auto load_step = [&](int tl, int ps, uint32_t (&d)[G::kWords]) {
-        const int c = min(ps * waves + wave, chunks - 1);
+        const int c = min(ps * span + gwave, chunks - 1);
         load_blocks<LAYOUT, NB>(t, col_base + min(tl, tiles - 1) * 16 + (lane & 15),
                                 c * G::kUnits + (lane >> 4) * NB / 8, half, d);
     };
     uint32_t wr[G::kWords], wn[G::kWords];
-    load_step(0, 0, wr);
+    load_step(tile, 0, wr);
     __builtin_amdgcn_sched_barrier(0);
     if (wave < chunks) stage(wave);
     __syncthreads();
 
     auto step = [&](const uint32_t (&d)[G::kWords], uint32_t (&next)[G::kWords]) {
-        const int nt = pass + 1 < passes ? tile : tile + 1, np = pass + 1 < passes ? pass + 1 : 0;
+        const int nt = pass + 1 < passes ? tile : tile + groups, np = pass + 1 < passes ? pass + 1 : 0;
         load_step(nt, np, next);
-        const int first = pass * waves, mine = first + wave;
+        const int first = pass * span, mine = GROUPS && (group >= groups || tile >= tiles) ? chunks : first + gwave;
         float terms[RPL][G::kChunk];
         uint32_t w[36];
         lane_words<LAYOUT, NB>(d, half, w);
         if (mine < chunks) chunk_terms<RPL, NB>(w, lds + static_cast<size_t>(mine) * G::kChunkBytes, terms);
         // The waves add their terms in turn, in block order.
-        const int active = min(waves, chunks - first);
+        const int active = min(span, chunks - first);
         for (int turn = 0; turn < active; ++turn) {
-            if (turn == wave) {
+            if (GROUPS ? turn + first == mine : turn == wave) {
                 float acc[RPL];
 #pragma unroll
                 for (int i = 0; i < RPL; ++i) acc[i] = mine == 0 ? 0.0f : run[i * 64 + lane];
@@ -421,22 +431,22 @@ __global__ __launch_bounds__(64 * kWaves<NB>) void q4_0_rows_kernel(Q4Task t) {
 
 constexpr int kBatchBlocks = 8;  // NB of the batch kernels
 
-template <int LAYOUT, bool X>
+template <int LAYOUT, bool X, bool GROUPS>
 __device__ __forceinline__ void rows_batch_item(const Q4Task &t, int col_base, int ncols) {
     if (LAYOUT == kLaneLayout || (LAYOUT == kEitherLayout && t.lanes))
-        rows_item<1, kLaneLayout, kBatchBlocks, X>(t, 0, col_base, ncols);
+        rows_item<1, kLaneLayout, kBatchBlocks, X, GROUPS>(t, 0, col_base, ncols);
     else
-        rows_item<1, kNativeRows, kBatchBlocks, X>(t, 0, col_base, ncols);
+        rows_item<1, kNativeRows, kBatchBlocks, X, GROUPS>(t, 0, col_base, ncols);
 }
 
-template <int LAYOUT, bool X>
+template <int LAYOUT, bool X, bool GROUPS>
 __global__ __launch_bounds__(64 * kWaves<kBatchBlocks>) void q4_0_rows_batch_kernel(const Q4Task *__restrict__ tasks,
                                                                                     const Q4Item *__restrict__ items) {
     const Q4Item item = items[blockIdx.x];
-    rows_batch_item<LAYOUT, X>(tasks[item.task], item.col_base, item.ncols);
+    rows_batch_item<LAYOUT, X, GROUPS>(tasks[item.task], item.col_base, item.ncols);
 }
 
-template <int LAYOUT, bool X>
+template <int LAYOUT, bool X, bool GROUPS>
 __global__ __launch_bounds__(64 * kWaves<kBatchBlocks>) void q4_0_rows_arg_batch_kernel(Q4ArgBatch a) {
     const int i = static_cast<int>(blockIdx.x);
     int ti = 0;
@@ -444,26 +454,7 @@ __global__ __launch_bounds__(64 * kWaves<kBatchBlocks>) void q4_0_rows_arg_batch
     for (int j = 1; j < kArgTasks; ++j) ti += i >= a.first_item[j] ? 1 : 0;
     const Q4Task t = a.task[ti];
     const int col_base = (i - a.first_item[ti]) * t.cpw;
-    rows_batch_item<LAYOUT, X>(t, col_base, min(t.cpw, t.ncols - col_base));
-}
-
-// Waves per workgroup for `chunks` chunks of K: as few passes as fit.
-template <int NB>
-int waves_of(int chunks) {
-    const int passes = (chunks + kWaves<NB> - 1) / kWaves<NB>;
-    return (chunks + passes - 1) / passes;
-}
-
-// Columns per workgroup (16-column tiles that share a staged activation): one
-// tile while the chip holds every workgroup at once, two where that makes one
-// round of them, and for larger grids up to three as long as several rounds
-// remain to even out the last.
-int columns_per_workgroup(long tiles, int waves, int waves_per_cu, size_t lds) {
-    const long per_cu = std::max<long>(1, std::min<long>(waves_per_cu / waves, static_cast<long>(kLds / lds)));
-    const long slots = compute_units() * per_cu;
-    if (tiles <= slots) return 16;
-    if (tiles <= 2 * slots) return 32;
-    return 16 * static_cast<int>(std::min<long>(3, std::max<long>(1, tiles / (4 * slots))));
+    rows_batch_item<LAYOUT, X, GROUPS>(t, col_base, min(t.cpw, t.ncols - col_base));
 }
 
 template <int NB>
@@ -474,10 +465,11 @@ int chunks_of(int blocks) {
 template <int RPL, int NB>
 int launch_rows(Q4Task t, hipStream_t stream) {
     const int chunks = chunks_of<NB>(t.blocks);
-    const int waves = waves_of<NB>(chunks);
+    const int waves = rows_waves(chunks, kWaves<NB>);
     const int groups = (t.rows + 4 * RPL - 1) / (4 * RPL);
     const size_t lds = RowsGeo<RPL, NB>::bytes(chunks);
-    t.cpw = columns_per_workgroup(static_cast<long>(groups) * ((t.ncols + 15) / 16), waves, NB == 8 ? 12 : 16, lds);
+    t.cpw = 16 * rows_steps(static_cast<long>(groups) * ((t.ncols + 15) / 16),
+                            compute_units() * rows_resident(waves, NB == 8 ? kRowsWavesPerCu : 16, lds));
     const dim3 grid((t.ncols + t.cpw - 1) / t.cpw, groups, 1);
     return t.lanes ? launch("q4_0_linear_kernel", q4_0_rows_kernel<RPL, kLaneLayout, NB>, grid, dim3(64 * waves), lds,
                             stream, t)
@@ -488,7 +480,7 @@ int launch_rows(Q4Task t, hipStream_t stream) {
 template <int RPL, int NB>
 bool fits(int blocks) {
     const int chunks = chunks_of<NB>(blocks);
-    return chunks <= kWaves<NB> * kMaxPasses && RowsGeo<RPL, NB>::bytes(chunks) <= kLds;
+    return chunks <= kWaves<NB> * kMaxPasses && RowsGeo<RPL, NB>::bytes(chunks) <= kRowsLds;
 }
 
 // The LDS of both chunk sizes, so that a shape fits or not by its rows and K.
@@ -598,27 +590,37 @@ int q4_0_rows_linear(const Q4Task &t, hipStream_t stream) {
     }
 }
 
-bool q4_0_rows_batch_supported(const Q4Task &t) { return layout_ok(t) && t.rows <= 4 && fits(t.blocks, 1); }
+static_assert(RowsGeo<1, kBatchBlocks>::kChunkBytes == kRowsChunkBytes && kWaves<kBatchBlocks> == kRowsWaves &&
+                  kMaxPasses == kRowsMaxPasses,
+              "the plan's figures of a chunk and a workgroup");
 
-int q4_0_rows_plan(Q4Task *tasks, uint32_t count, size_t *lds) {
-    int least = 1 << 30, most = 1;
-    long tiles = 0;
-    size_t bytes = 0;
+static RowsTiles tiles_by_chunks(const Q4Task *tasks, uint32_t count) {
+    RowsTiles tiles;
+    for (uint32_t i = 0; i < count; ++i)
+        tiles[chunks_of<kBatchBlocks>(tasks[i].blocks)] += (static_cast<long>(tasks[i].ncols) + 15) / 16;
+    return tiles;
+}
+
+bool q4_0_rows_batch_takes(const Q4Task *tasks, uint32_t count) {
+    double units = 0.0, columns = 0.0;
+    bool fp32 = false;
     for (uint32_t i = 0; i < count; ++i) {
-        const int chunks = chunks_of<kBatchBlocks>(tasks[i].blocks);
-        least = std::min(least, waves_of<kBatchBlocks>(chunks));
-        most = std::max(most, chunks);
-        bytes = std::max(bytes, RowsGeo<1, kBatchBlocks>::bytes(chunks));
-        tiles += (tasks[i].ncols + 15) / 16;
+        Q4Task t = tasks[i];
+        fp32 = fp32 || t.x != nullptr;
+        t.x = nullptr;
+        if (t.rows > 4 || !layout_ok(t) || !fits(t.blocks, 1)) return false;
+        units += t.blocks / 8.0 * t.ncols;
+        columns += t.ncols;
     }
-    // The waves that the shortest K needs (a longer one takes more passes):
-    // waves without a chunk would idle.  K = 2048 and 5632 together, the
-    // 154-linear step at two rows: six waves 222 us, two 139.
-    const int waves = std::max(least, (most + kMaxPasses - 1) / kMaxPasses);
-    const int cpw = columns_per_workgroup(tiles, waves, 12, bytes);
-    for (uint32_t i = 0; i < count; ++i) tasks[i].cpw = std::min(cpw, (tasks[i].ncols + 15) / 16 * 16);
-    *lds = bytes;
-    return 64 * waves;
+    if (columns > 16.0 * (1 << 24)) return false;  // a table of one item per 16 columns
+    return rows_batch_preferred(tiles_by_chunks(tasks, count), units, fp32, compute_units());
+}
+
+RowsPlan q4_0_rows_plan(Q4Task *tasks, uint32_t count) {
+    const RowsPlan plan = rows_batch_plan(tiles_by_chunks(tasks, count), compute_units());
+    for (uint32_t i = 0; i < count; ++i)
+        tasks[i].cpw = std::min(plan.columns(chunks_of<kBatchBlocks>(tasks[i].blocks)), (tasks[i].ncols + 15) / 16 * 16);
+    return plan;
 }
 
 namespace {
@@ -628,26 +630,30 @@ Kernel by_layout(int layout, Kernel lanes, Kernel native, Kernel either) {
     return layout == kLaneLayout ? lanes : layout == kNativeRows ? native : either;
 }
 
-template <bool X>
-int launch_batch(const Q4ArgBatch *args, const Q4Task *tasks, const Q4Item *items, uint32_t grid, int threads,
-                 size_t lds, int layout, hipStream_t stream) {
+template <bool X, bool GROUPS>
+int launch_batch(const Q4ArgBatch *args, const Q4Task *tasks, const Q4Item *items, uint32_t grid, const RowsPlan &plan,
+                 int layout, hipStream_t stream) {
+    const dim3 blocks(grid), threads(64 * plan.waves);
     if (args != nullptr)
         return launch("q4_0_batch_kernel",
-                      by_layout(layout, q4_0_rows_arg_batch_kernel<kLaneLayout, X>,
-                                q4_0_rows_arg_batch_kernel<kNativeRows, X>, q4_0_rows_arg_batch_kernel<kEitherLayout, X>),
-                      dim3(grid), dim3(threads), lds, stream, *args);
+                      by_layout(layout, q4_0_rows_arg_batch_kernel<kLaneLayout, X, GROUPS>,
+                                q4_0_rows_arg_batch_kernel<kNativeRows, X, GROUPS>,
+                                q4_0_rows_arg_batch_kernel<kEitherLayout, X, GROUPS>),
+                      blocks, threads, plan.lds, stream, *args);
     return launch("q4_0_batch_kernel",
-                  by_layout(layout, q4_0_rows_batch_kernel<kLaneLayout, X>, q4_0_rows_batch_kernel<kNativeRows, X>,
-                            q4_0_rows_batch_kernel<kEitherLayout, X>),
-                  dim3(grid), dim3(threads), lds, stream, tasks, items);
+                  by_layout(layout, q4_0_rows_batch_kernel<kLaneLayout, X, GROUPS>,
+                            q4_0_rows_batch_kernel<kNativeRows, X, GROUPS>,
+                            q4_0_rows_batch_kernel<kEitherLayout, X, GROUPS>),
+                  blocks, threads, plan.lds, stream, tasks, items);
 }
 
 }  // namespace
 
-int q4_0_rows_batch(const Q4ArgBatch *args, const Q4Task *tasks, const Q4Item *items, uint32_t grid, int threads,
-                    size_t lds, int layout, bool fp32_rows, hipStream_t stream) {
-    return fp32_rows ? launch_batch<true>(args, tasks, items, grid, threads, lds, layout, stream)
-                     : launch_batch<false>(args, tasks, items, grid, threads, lds, layout, stream);
+int q4_0_rows_batch(const Q4ArgBatch *args, const Q4Task *tasks, const Q4Item *items, uint32_t grid,
+                    const RowsPlan &plan, int layout, bool fp32_rows, hipStream_t stream) {
+    auto run = fp32_rows ? (plan.groups ? launch_batch<true, true> : launch_batch<true, false>)
+                         : (plan.groups ? launch_batch<false, true> : launch_batch<false, false>);
+    return run(args, tasks, items, grid, plan, layout, stream);
 }
 
 }  // namespace qxt

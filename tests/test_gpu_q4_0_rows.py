@@ -176,3 +176,46 @@ def test_row_tile_batch_captured_and_replayed_reads_the_rows_of_each_replay() ->
 ])
 def test_short_prompts_on_row_tiles_bit_exact(rows: int, blocks: int, n: int, wcol0: int, ncols: int) -> None:
     _check_linear("native", rows, blocks, n, wcol0, ncols)
+
+
+def _check_batch(shapes, source: str, layouts: str, offset: int = 0) -> None:
+    """One batch of (rows, blocks, columns) tasks; `offset` bytes before every native activation."""
+    rng = np.random.default_rng(len(shapes) * 1000 + len(source) + len(layouts))
+    tasks, checks = [], []
+    for i, (rows, blocks, n) in enumerate(shapes):
+        act, wt = _operands(int(rng.integers(1 << 30)), rows, blocks, n)
+        lanes = layouts == "lanes" or (layouts == "mixed" and i % 2 == 0)
+        task = {"weight": q4.pack_ggml_q4_0_lane_weights(dev(wt)) if lanes else dev(wt),
+                "destination": torch.full((rows, n + 3), -77.0, device="cuda"), "output_column_start": 2}
+        if source == "fp32" or (source == "mixed" and i % 2 == 0):
+            x = rng.standard_normal((rows, blocks * 32), dtype=np.float32)
+            act = oracle.quantize_q8_0_blocks(x)
+            task["x"] = dev(x)
+        else:
+            raw = torch.zeros(act.size + offset, dtype=torch.uint8, device="cuda")
+            raw[offset:] = dev(act).flatten()
+            task["activation"] = raw[offset:].view(act.shape)
+        tasks.append(task)
+        checks.append((act, wt))
+    with q4.Q4_0LinearBatch(tasks) as batch:
+        for _ in range(2):
+            batch.launch()
+        torch.cuda.synchronize()
+        for task, (act, wt) in zip(tasks, checks):
+            got = task["destination"].cpu().numpy()
+            n = wt.shape[0]
+            some = np.unique(np.concatenate([np.arange(min(n, 200)), np.arange(0, n, 67), np.arange(max(0, n - 200), n)]))
+            np.testing.assert_array_equal(got[:, 2 + some], oracle.q4_0_q8_0_reference(act, wt[some]))
+            np.testing.assert_array_equal(got[:, [0, 1, -1]], -77.0)
+
+
+@pytest.mark.parametrize("source", ["fp32", "native"])
+@pytest.mark.parametrize("layouts", ["lanes", "native", "mixed"])
+@pytest.mark.parametrize("shapes", [
+    # A long K beside short ones that fill the chip: several column tiles of a workgroup side by side.
+    [(4, 64, 5000), (2, 512, 40)],                                      # kernel arguments
+    [(2, 16, 4001), (3, 32, 3000), (4, 256, 130), (1, 64, 333), (2, 264, 50), (4, 16, 9)],  # device tables
+    [(3, 32, 9000), (2, 96, 2100), (4, 448, 17), (2, 32, 15)],          # waves past the last group
+])
+def test_row_tile_batch_of_short_and_long_k_bit_exact(shapes, layouts: str, source: str) -> None:
+    _check_batch(shapes, source, layouts)
