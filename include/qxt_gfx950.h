@@ -322,7 +322,8 @@ int qxt_q4_0_batch_prepare(const qxt_q4_0_task *tasks, uint32_t count, qxt_q4_0_
 
 /* Enqueue the whole batch on `stream`: the Q8_0 pre-pass (when a task has fp32
  * rows that the batch grid does not quantise itself) and the batch grid;
- * graph-capturable.
+ * graph-capturable.  Launches of one batch write the same outputs, and the
+ * pre-pass a buffer of the batch: order them (one stream, or events).
  * Replaces qpu_llama_q4_0_linear_submit (qpu_llama_q4_0.h:72-75). */
 int qxt_q4_0_batch_launch(const qxt_q4_0_batch *batch, void *stream);
 

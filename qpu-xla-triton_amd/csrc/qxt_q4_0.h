@@ -84,13 +84,13 @@ struct Q4ArgBatch {
 // Two or more rows on 16 x 16 matrix-core tiles (qxt_q4_0_rows.hip).  The
 // single linear returns QXT_CAPABILITY_MISSING (no message, nothing launched)
 // for shapes it does not take.  The batch takes tasks of at most four rows each,
-// all native Q8_0 or (fp32_rows) all fp32, planned by q4_0_rows_plan (which
-// sets every task's cpw); `args` or, when that is null, the device tables
-// `tasks` and `items`.
+// planned by q4_0_rows_plan (which sets every task's cpw), whose activations are
+// `source`; `args` or, when that is null, the device tables `tasks` and `items`.
+enum RowsSource { kRowsQ8 = 0, kRowsFp32 = 1, kRowsEither = 2 };  // kRowsEither: fp32 where the task's x is set
 int q4_0_rows_linear(const Q4Task &t, hipStream_t stream);
 bool q4_0_rows_batch_takes(const Q4Task *tasks, uint32_t count);
 RowsPlan q4_0_rows_plan(Q4Task *tasks, uint32_t count);
 int q4_0_rows_batch(const Q4ArgBatch *args, const Q4Task *tasks, const Q4Item *items, uint32_t grid,
-                    const RowsPlan &plan, int layout, bool fp32_rows, hipStream_t stream);
+                    const RowsPlan &plan, int layout, RowsSource source, hipStream_t stream);
 
 }  // namespace qxt

@@ -1450,7 +1450,7 @@ struct qxt_q4_0_batch {
     size_t lds = 0;
     bool rows = false;     // the row-tile kernels (tasks of two to four rows), by rows_plan
     RowsPlan rows_plan{};
-    bool rows_fp32 = false;  // they quantise fp32 rows themselves
+    RowsSource rows_source = kRowsQ8;
     bool in_args = false;  // tasks and items travel in the kernel arguments
     Q4ArgBatch args{};
 };
@@ -1764,8 +1764,8 @@ int qxt_q4_0_batch_prepare(const qxt_q4_0_task *tasks, uint32_t count, qxt_q4_0_
     // tiles were narrowed (too few columns to fill the chip) runs it with
     // kPrefetchUnits units per thread, its tiles planned for that.
     // Batches with tasks of two to four rows mostly run the row-tile kernels,
-    // which quantise fp32 rows themselves when every task of a small batch
-    // gives them and read the pre-pass's Q8_0 rows otherwise.
+    // which quantise the fp32 rows of a small batch themselves and read the
+    // pre-pass's Q8_0 rows otherwise.
     const bool row_tiles = mr != 1 && q4_0_rows_batch_takes(host.data(), count);
     if (row_tiles) {
         // Long K first: a last round of workgroups that each take several
@@ -1786,15 +1786,16 @@ int qxt_q4_0_batch_prepare(const qxt_q4_0_task *tasks, uint32_t count, qxt_q4_0_
     if (!small && !kPrefetchLargeBatches) prefetch_candidate = false;
     // Every other small batch quantises its fp32 rows inside each workgroup
     // too (an L2-resident re-read per workgroup) rather than waiting for a
-    // separate pre-pass launch; larger ones run the pre-pass.
-    // (Up to eight column tiles per CU: the 16-stage step of four rows over
-    // K = 4096 / 11008 layers, fused 239, pre-pass 268 us; whole-step batches of
-    // thousands of tiles, pre-pass 134, fused 154 us.)
+    // separate pre-pass launch; larger ones run the pre-pass.  A batch without
+    // a pre-pass has no memory that its launches write besides the outputs.
+    // (Row tiles also up to eight column tiles per CU: the 16-stage step of
+    // four rows over K = 4096 / 11008 layers, fused 239, pre-pass 268 us;
+    // whole-step batches of thousands of tiles, pre-pass 134, fused 154 us.)
     uint64_t row_tile_count = 0;
     for (uint32_t i = 0; i < count; ++i) row_tile_count += (static_cast<uint64_t>(host[i].ncols) + 15) / 16;
-    const bool rows_fp32 =
-        row_tiles && jobs.size() == count && row_tile_count <= 8ull * static_cast<uint64_t>(compute_units());
-    const bool fused = row_tiles ? rows_fp32 : small || prefetch_candidate;
+    const bool fused = small || prefetch_candidate ||
+                       (row_tiles && row_tile_count <= 8ull * static_cast<uint64_t>(compute_units()));
+    const RowsSource rows_source = jobs.empty() || !fused ? kRowsQ8 : jobs.size() == count ? kRowsFp32 : kRowsEither;
     const bool narrowed = max_cpw < (1 << 30);
     const int upt = prefetch_candidate && narrowed ? kPrefetchUnits : units_per_thread(mr);
     if (upt != units_per_thread(mr)) {
@@ -1901,7 +1902,7 @@ int qxt_q4_0_batch_prepare(const qxt_q4_0_task *tasks, uint32_t count, qxt_q4_0_
     batch->grid = static_cast<uint32_t>(items.size());
     batch->mr = mr;
     batch->rows = row_tiles;
-    batch->rows_fp32 = rows_fp32;
+    batch->rows_source = rows_source;
     batch->rows_plan = rows_plan;
     batch->layout = layout;
     // The prefetch kernel runs exactly the batches planned for it.
@@ -1967,7 +1968,7 @@ int qxt_q4_0_batch_launch(const qxt_q4_0_batch *batch, void *stream) {
     }
     if (batch->rows)
         return q4_0_rows_batch(batch->in_args ? &batch->args : nullptr, batch->tasks, batch->items, batch->grid,
-                               batch->rows_plan, batch->layout, batch->rows_fp32, as_stream(stream));
+                               batch->rows_plan, batch->layout, batch->rows_source, as_stream(stream));
     const BatchKernel kernel =
         batch_kernel(batch->mr, batch->layout, batch->prefetch, batch->upt, batch->split, batch->threads);
     const dim3 block(batch->threads);

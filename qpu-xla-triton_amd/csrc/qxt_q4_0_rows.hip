@@ -431,22 +431,27 @@ __global__ __launch_bounds__(64 * kWaves<NB>) void q4_0_rows_kernel(Q4Task t) {
 
 constexpr int kBatchBlocks = 8;  // NB of the batch kernels
 
-template <int LAYOUT, bool X, bool GROUPS>
+template <int LAYOUT, int SOURCE, bool GROUPS>
 __device__ __forceinline__ void rows_batch_item(const Q4Task &t, int col_base, int ncols) {
-    if (LAYOUT == kLaneLayout || (LAYOUT == kEitherLayout && t.lanes))
-        rows_item<1, kLaneLayout, kBatchBlocks, X, GROUPS>(t, 0, col_base, ncols);
-    else
-        rows_item<1, kNativeRows, kBatchBlocks, X, GROUPS>(t, 0, col_base, ncols);
+    auto run = [&](auto x) {
+        constexpr bool X = decltype(x)::value;
+        if (LAYOUT == kLaneLayout || (LAYOUT == kEitherLayout && t.lanes))
+            rows_item<1, kLaneLayout, kBatchBlocks, X, GROUPS>(t, 0, col_base, ncols);
+        else
+            rows_item<1, kNativeRows, kBatchBlocks, X, GROUPS>(t, 0, col_base, ncols);
+    };
+    if (SOURCE == kRowsFp32 || (SOURCE == kRowsEither && t.x != nullptr)) run(std::true_type{});
+    else run(std::false_type{});
 }
 
-template <int LAYOUT, bool X, bool GROUPS>
+template <int LAYOUT, int SOURCE, bool GROUPS>
 __global__ __launch_bounds__(64 * kWaves<kBatchBlocks>) void q4_0_rows_batch_kernel(const Q4Task *__restrict__ tasks,
                                                                                     const Q4Item *__restrict__ items) {
     const Q4Item item = items[blockIdx.x];
-    rows_batch_item<LAYOUT, X, GROUPS>(tasks[item.task], item.col_base, item.ncols);
+    rows_batch_item<LAYOUT, SOURCE, GROUPS>(tasks[item.task], item.col_base, item.ncols);
 }
 
-template <int LAYOUT, bool X, bool GROUPS>
+template <int LAYOUT, int SOURCE, bool GROUPS>
 __global__ __launch_bounds__(64 * kWaves<kBatchBlocks>) void q4_0_rows_arg_batch_kernel(Q4ArgBatch a) {
     const int i = static_cast<int>(blockIdx.x);
     int ti = 0;
@@ -454,7 +459,7 @@ __global__ __launch_bounds__(64 * kWaves<kBatchBlocks>) void q4_0_rows_arg_batch
     for (int j = 1; j < kArgTasks; ++j) ti += i >= a.first_item[j] ? 1 : 0;
     const Q4Task t = a.task[ti];
     const int col_base = (i - a.first_item[ti]) * t.cpw;
-    rows_batch_item<LAYOUT, X, GROUPS>(t, col_base, min(t.cpw, t.ncols - col_base));
+    rows_batch_item<LAYOUT, SOURCE, GROUPS>(t, col_base, min(t.cpw, t.ncols - col_base));
 }
 
 template <int NB>
@@ -625,35 +630,40 @@ RowsPlan q4_0_rows_plan(Q4Task *tasks, uint32_t count) {
 
 namespace {
 
-template <typename Kernel>
-Kernel by_layout(int layout, Kernel lanes, Kernel native, Kernel either) {
-    return layout == kLaneLayout ? lanes : layout == kNativeRows ? native : either;
-}
-
-template <bool X, bool GROUPS>
+// Mixed sources have one instantiation for every layout.
+template <int SOURCE, bool GROUPS>
 int launch_batch(const Q4ArgBatch *args, const Q4Task *tasks, const Q4Item *items, uint32_t grid, const RowsPlan &plan,
                  int layout, hipStream_t stream) {
     const dim3 blocks(grid), threads(64 * plan.waves);
-    if (args != nullptr)
-        return launch("q4_0_batch_kernel",
-                      by_layout(layout, q4_0_rows_arg_batch_kernel<kLaneLayout, X, GROUPS>,
-                                q4_0_rows_arg_batch_kernel<kNativeRows, X, GROUPS>,
-                                q4_0_rows_arg_batch_kernel<kEitherLayout, X, GROUPS>),
-                      blocks, threads, plan.lds, stream, *args);
-    return launch("q4_0_batch_kernel",
-                  by_layout(layout, q4_0_rows_batch_kernel<kLaneLayout, X, GROUPS>,
-                            q4_0_rows_batch_kernel<kNativeRows, X, GROUPS>,
-                            q4_0_rows_batch_kernel<kEitherLayout, X, GROUPS>),
-                  blocks, threads, plan.lds, stream, tasks, items);
+    auto run = [&](auto lc) {
+        constexpr int L = decltype(lc)::value;
+        return args != nullptr ? launch("q4_0_batch_kernel", q4_0_rows_arg_batch_kernel<L, SOURCE, GROUPS>, blocks,
+                                        threads, plan.lds, stream, *args)
+                               : launch("q4_0_batch_kernel", q4_0_rows_batch_kernel<L, SOURCE, GROUPS>, blocks, threads,
+                                        plan.lds, stream, tasks, items);
+    };
+    if constexpr (SOURCE != kRowsEither) {
+        if (layout == kLaneLayout) return run(std::integral_constant<int, kLaneLayout>{});
+        if (layout == kNativeRows) return run(std::integral_constant<int, kNativeRows>{});
+    }
+    return run(std::integral_constant<int, kEitherLayout>{});
+}
+
+template <bool GROUPS>
+int launch_batch(const Q4ArgBatch *args, const Q4Task *tasks, const Q4Item *items, uint32_t grid, const RowsPlan &plan,
+                 int layout, RowsSource source, hipStream_t stream) {
+    return source == kRowsQ8 ? launch_batch<kRowsQ8, GROUPS>(args, tasks, items, grid, plan, layout, stream)
+           : source == kRowsFp32
+               ? launch_batch<kRowsFp32, GROUPS>(args, tasks, items, grid, plan, layout, stream)
+               : launch_batch<kRowsEither, GROUPS>(args, tasks, items, grid, plan, layout, stream);
 }
 
 }  // namespace
 
 int q4_0_rows_batch(const Q4ArgBatch *args, const Q4Task *tasks, const Q4Item *items, uint32_t grid,
-                    const RowsPlan &plan, int layout, bool fp32_rows, hipStream_t stream) {
-    auto run = fp32_rows ? (plan.groups ? launch_batch<true, true> : launch_batch<true, false>)
-                         : (plan.groups ? launch_batch<false, true> : launch_batch<false, false>);
-    return run(args, tasks, items, grid, plan, layout, stream);
+                    const RowsPlan &plan, int layout, RowsSource source, hipStream_t stream) {
+    return plan.groups ? launch_batch<true>(args, tasks, items, grid, plan, layout, source, stream)
+                       : launch_batch<false>(args, tasks, items, grid, plan, layout, source, stream);
 }
 
 }  // namespace qxt

@@ -11,6 +11,7 @@ import pytest
 import torch
 
 import oracle
+from qpu_xla_amd import _lib
 from qpu_xla_amd.kernels import ggml_q4_0 as q4
 
 pytestmark = pytest.mark.gpu
@@ -209,7 +210,7 @@ def _check_batch(shapes, source: str, layouts: str, offset: int = 0) -> None:
             np.testing.assert_array_equal(got[:, [0, 1, -1]], -77.0)
 
 
-@pytest.mark.parametrize("source", ["fp32", "native"])
+@pytest.mark.parametrize("source", ["fp32", "native", "mixed"])
 @pytest.mark.parametrize("layouts", ["lanes", "native", "mixed"])
 @pytest.mark.parametrize("shapes", [
     # A long K beside short ones that fill the chip: several column tiles of a workgroup side by side.
@@ -219,3 +220,16 @@ def _check_batch(shapes, source: str, layouts: str, offset: int = 0) -> None:
 ])
 def test_row_tile_batch_of_short_and_long_k_bit_exact(shapes, layouts: str, source: str) -> None:
     _check_batch(shapes, source, layouts)
+
+
+@pytest.mark.parametrize("shapes", [
+    [(2, 64, 700), (4, 40, 130)],                                   # kernel arguments
+    [(3, 32, 9000), (2, 96, 2100), (4, 448, 17), (2, 32, 15), (1, 8, 40)],  # device tables, tiles side by side
+    [(2, 128, 300)] * 5,
+])
+def test_small_batch_of_mixed_activations_is_one_launch(shapes) -> None:
+    # fp32 rows beside native ones are quantised in the workgroups: no pre-pass, no buffer that launches share.
+    with _lib.launch_timing() as timing:
+        _check_batch(shapes, "mixed", "mixed")
+    names = [name for name, _ in timing.records if "pack" not in name]
+    assert names == ["q4_0_batch_kernel"] * 2
