@@ -33,7 +33,7 @@
 // chunk of 32 blocks at one row per lane, 6 to 7 cycles each with one wave per
 // SIMD) and the waves' turns; large grids, those instructions on every SIMD.
 // Measured on MI355X against the kernels it replaces (bit-identical): single
-// linears in takes() below; a staged decode step of four rows over Llama-7B
+// linears at rows_linear_takes (qxt_q4_0_rows_plan.h); a staged decode step of four rows over Llama-7B
 // class layers (K = 4096 / 11008, 16 stages) 557 -> 239 us; whole-step batches of
 // four rows 387 -> 122 us (the same four layers, two launches) and 196 -> 139 us
 // (154 TinyLlama linears).
@@ -509,48 +509,6 @@ bool layout_ok(const Q4Task &t) {
 
 }  // namespace
 
-// Which single linears take the row tiles, by what was measured faster on
-// MI355X (us, the other kernels -> these; back to back over rotated weights).
-// The other kernels: q4_0_mfma4 (four-row tiles, K <= 4096 with 16 % (K / 256)
-// == 0), q4_0_stream (native rows, blocks over lanes), v_dot4 tiles.
-static bool takes(const Q4Task &t, long tiles, long cus) {
-    const int blocks = t.blocks;
-    const bool mfma4 = blocks <= 128 && 16 % (blocks / 8) == 0;
-    if (t.lanes) {
-        if (t.rows <= 3) {
-            // 2048 x 256 4.3 -> 3.3, 2048 x 8192 5.9 -> 5.6, but x 32000 10.9 -> 12.0;
-            // 4096 x 4096 6.4 -> 5.7, x 4608 6.6 -> 7.8; 5632 x 2048 6.9 -> 6.4,
-            // 11008 x 4096 15.8 -> 12.5, but x 2048 9.3 -> 11.7, 8192 x 1024 6.7 -> 7.9.
-            if (blocks <= 64) return tiles <= 2 * cus;
-            if (blocks <= 128) return tiles <= cus;
-            return blocks <= 224 || tiles >= cus;
-        }
-        if (t.rows == 4) {
-            // 2048 x 256 4.3 -> 3.4, 4096 x 4096 5.3 -> 5.7; 5632 x 2048 7.3 -> 6.4,
-            // 8192 x 4096 10.8 -> 9.5, but x 1024 7.6 -> 7.9.
-            if (mfma4) return 2 * tiles <= cus;
-            return blocks <= 224 || 2 * tiles >= cus;
-        }
-        // 8 rows: 4096 x 4096 7.0 -> 6.4, x 11008 18.2 -> 12.2, x 6000 8.0 -> 9.5;
-        // 2048 x 5632 6.1 -> 5.9; 11008 x 4096 32.1 -> 14.6.
-        return !(mfma4 && blocks > 64 && t.rows <= 8 && tiles > cus && tiles <= 2 * cus);
-    }
-    if (t.rows <= 4) {
-        // Two to four rows, native: 2048 x 256 4.2 -> 3.2, x 5632 5.6 -> 4.8; 4 rows
-        // 2304 x 6000 6.9 -> 5.4, 11008 x 4096 13.4 -> 11.4, but x 2048 10.4 -> 11.1,
-        // 4096 x 4608 6.6 -> 8.4; 2 rows 5632 x 2048 5.1 -> 6.4.
-        if (blocks <= 64) return tiles <= 2 * cus;
-        if (t.rows < 4) return false;
-        return blocks > 256 ? tiles >= cus : blocks <= 128 && !mfma4 && tiles <= 2 * cus;
-    }
-    // 8 rows, native: 2048 x 5632 6.2 -> 5.6, 4096 x 4096 7.5 -> 6.1, 4096 x 11008
-    // 16.0 -> 12.7, 11008 x 4096 22.3 -> 13.0, but 4096 x 4608 8.1 -> 8.8, 8192 x 1024
-    // 6.9 -> 9.1, x 2048 8.2 -> 9.2, 14336 x 1024 10.1 -> 13.3.
-    if (blocks > 192 && 4 * tiles <= cus) return false;
-    if (blocks > 224 && blocks <= 256 && tiles < cus && t.rows <= 8) return false;
-    return !(blocks > 64 && blocks <= 128 && tiles > cus && 4 * tiles <= 5 * cus);
-}
-
 // Sixteen or more native rows: row groups of this kernel against the 64 x 64
 // prefill tiles (qxt_q4_0_tiled.hip), whose time is the K of one tile until
 // their grid fills the chip.  Both from sweeps on MI355X (us): this kernel 2.5 +
@@ -571,7 +529,7 @@ static bool takes_prefill(const Q4Task &t, long tiles) {
 int q4_0_rows_linear(const Q4Task &t, hipStream_t stream) {
     if (t.rows < 2 || !layout_ok(t)) return QXT_CAPABILITY_MISSING;
     const long tiles = (t.ncols + 15) / 16, cus = compute_units();
-    if (t.rows > 15 ? !takes_prefill(t, tiles) : !takes(t, tiles, cus)) return QXT_CAPABILITY_MISSING;
+    if (t.rows > 15 ? !takes_prefill(t, tiles) : !rows_linear_takes(t.lanes != 0, t.rows, t.blocks, tiles, cus)) return QXT_CAPABILITY_MISSING;
     // The fewest rows per lane that leave every workgroup a CU of its own;
     // larger grids take all rows at once (K = 5632, N = 2048, 5 rows: two row
     // groups 6.4 us, one 7.0; K = 2048, N = 5632: 6.6 and 5.3).

@@ -1,6 +1,6 @@
-// Launch plan of a batch on the row tiles (qxt_q4_0_rows.hip): waves of a
-// workgroup, LDS, and column tiles per workgroup by the length of K.  Host
-// code only, without HIP.
+// Which linears and batches run on the row tiles (qxt_q4_0_rows.hip), and the
+// launch plan of a batch: waves of a workgroup, LDS, and column tiles per
+// workgroup by the length of K.  Host code only, without HIP.
 #pragma once
 
 #include <algorithm>
@@ -144,6 +144,79 @@ inline RowsPlan rows_batch_plan(const RowsTiles &tiles, int cus) {
     plan.evened = true;
     plan.evened = workgroups() <= slots;
     return plan;
+}
+
+// Which single linears of 2 to 15 rows take the row tiles, by what was measured
+// faster on MI355X (us, the other kernels -> these; back to back over rotated
+// weights).  Fitted to 8,100 shapes (25 K from 256 to 16384 x 18 N from 64 to
+// 32000 x 9 row counts x both layouts): 1.36 times the others in the geometric
+// mean, ten shapes more than 4 % slower, by at most 1.07, where taking every shape
+// leaves 1,588; on 3,360 others 1.34 times, 13 slower, by at most 1.35 (4 rows,
+// lanes, 6400 x 9216).  K x N below; `n` is column tiles per 256 CUs.  The other
+// kernels: q4_0_mfma4 (four-row tiles, K <= 4096 with 16 % (K / 256) == 0),
+// q4_0_stream (native rows, blocks over lanes), v_dot4 tiles.
+//   * Many tiles: the others stream the weights with more of them in flight,
+//     these are bound by instructions (lanes, 2 rows, 4608 x 32000 21.3 -> 45.2;
+//     but from K = 14336 their staged rows leave them one workgroup a CU:
+//     16384 x 8192 39.2 -> 26.3).
+//   * Just over one tile per CU these take a second round (lanes, 3 rows,
+//     4608 x 4608 8.4 -> 12.0; native, 4 rows, 14336 x 4608 15.7 -> 23.4).
+//   * Few tiles over a long K: the others spread it over the chip, these keep it
+//     to a workgroup per 16 columns (native, 5 rows, 8192 x 1024 6.9 -> 9.1,
+//     6144 x 64 3.9 -> 6.9; lanes 14336 x 64 9.0 -> 11.1).
+inline bool rows_linear_takes(bool lanes, int rows, int blocks, long tiles, long cus) {
+    const int b = blocks;
+    const long n = tiles * 256 / cus;
+    const bool mfma4 = b <= 128 && 16 % (b / 8) == 0;
+    const bool just_over = n > 256 && n <= 320;
+    const bool three = rows > 8 && rows <= 12;  // three rows a lane, the others' third round of four
+    if (b < 16 && n > 512) return three;        // three quarters of each chunk are empty
+    if (lanes) {
+        if (rows <= 3) {
+            // 2048 x 256 4.3 -> 3.3, 2048 x 8192 5.9 -> 5.6; 4096 x 4096 6.4 -> 5.7; 2 rows
+            // 5632 x 2048 6.9 -> 6.4, 11008 x 4096 15.8 -> 12.5; 3 rows 8192 x 8192 19.1 -> 15.1.
+            if (b <= 64) return n <= 512;
+            if (b <= (rows == 2 ? 176 : 224)) return n <= 256 || (b > 192 && n > 320 && n <= 512);
+            if (rows == 2) return b >= 448 ? n >= 192 : b > 256 && n > 192 && n <= 256;
+            return b >= 256 && n >= 256 && !(b <= 352 && just_over);
+        }
+        if (rows == 4) {
+            // 2048 x 256 4.3 -> 3.4, 2304 x 6000 6.9 -> 5.4, 5632 x 2048 7.3 -> 6.4,
+            // 5120 x 16384 28.5 -> 20.7, 8192 x 4096 10.8 -> 9.5.
+            if (mfma4) return n <= (b <= 64 ? 128 : 32);
+            if (b <= 128) return true;
+            if (b <= 192) return n <= 256 || (b >= 160 && n > (b == 192 ? 640 : 768) && n <= 1280);
+            return (b <= 224 || n >= 128) && !(b <= 352 && just_over);
+        }
+        // 8 rows: 4096 x 4096 7.0 -> 6.4, x 11008 18.2 -> 12.2, 2048 x 5632 6.1 -> 5.9,
+        // 2048 x 16384 8.8 -> 9.8 (not taken), 11008 x 4096 32.1 -> 14.6.
+        if (b >= 256 && n <= (rows <= 8 ? 32 : three ? 14 : 16)) return false;
+        if (rows <= 8 && b == 64) return n <= 512 || n > 1024;
+        if (rows <= 8 && b == 128) return n <= 256 || n > 512;
+        return !(rows <= 8 && b > 128 && b <= 192 && just_over);
+    }
+    if (rows <= 4) {
+        // 2048 x 256 4.2 -> 3.2, x 5632 5.6 -> 4.8; 4 rows 11008 x 4096 13.4 -> 11.4,
+        // but x 4608 14.7 -> 18.0 (not taken).
+        if (b <= 64) return n <= 512;
+        if (rows < 4) return false;
+        if (b <= 128) return !mfma4 && n <= 512;
+        return b > 256 && b < 416 && n >= 256 && !(n > 256 && n <= 358);
+    }
+    // 8 rows: 2048 x 5632 6.2 -> 5.6, 4096 x 4096 7.5 -> 6.1, x 11008 16.0 -> 12.7,
+    // 11008 x 4096 22.3 -> 13.0; 9 rows 14336 x 4608 35.3 -> 42.4 (not taken).
+    if (b <= 64) return true;
+    if (b > 496 && !(rows > 12 && n <= 256)) return false;
+    if (b >= 416 && three && n > 256 && n < 1024) return false;
+    if (just_over && (b <= 128 || (rows <= 8 && b >= 192 && b <= 216) || (three && b >= 336))) return false;
+    // Least tiles, by K, up to eight rows and past them.
+    const bool few = rows <= 8;
+    if (b <= 112) return n >= (few ? 32 : 16);
+    if (b <= 176) return n >= (few ? 96 : 64);
+    if (b <= 224) return n >= (few ? 128 : 96);
+    if (b <= 256) return n >= (few ? 256 : 128);
+    if (b < 416) return n >= (few ? 128 : 64);
+    return n >= (few ? 192 : 96);
 }
 
 }  // namespace qxt

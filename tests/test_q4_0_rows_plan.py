@@ -1,4 +1,4 @@
-"""The launch plan of a batch on the 16-row tiles, compiled for the host and checked without a GPU.
+"""The rules and the launch plan of the 16-row tiles, compiled for the host and checked without a GPU.
 
 A batch has one LDS size and one workgroup size, so tasks of a short K share
 the chip with the needs of the longest: the plan has to keep the waves of
@@ -29,6 +29,9 @@ extern "C" int plan(const int *chunks, const long *tiles, int n, int cus, double
     out[0] = p.waves, out[1] = static_cast<long>(p.lds), out[2] = p.groups, out[3] = p.steps;
     for (int i = 0; i < n; ++i) out[4 + i] = p.columns(chunks[i]);
     return qxt::rows_batch_preferred(t, units, fp32, cus);
+}
+extern "C" int linear_takes(int lanes, int rows, int blocks, long tiles, long cus) {
+    return qxt::rows_linear_takes(lanes, rows, blocks, tiles, cus);
 }
 """
 
@@ -128,3 +131,38 @@ def test_small_grids_of_a_longer_k_take_it_in_one_pass(library) -> None:
 ])
 def test_which_batches_take_the_row_tiles(library, shapes, fp32: bool, preferred: bool) -> None:
     assert _plan(library, shapes, fp32)[2] is preferred
+
+
+@pytest.mark.parametrize("layout,rows,k,n,taken", [
+    # Measured on MI355X: the other kernels / the row tiles, us.
+    ("lanes", 2, 4608, 32000, False),   # 21.3 / 45.3
+    ("lanes", 2, 5632, 11008, False),   # 12.9 / 21.3
+    ("lanes", 2, 5632, 4608, False),    # 8.7 / 13.1
+    ("lanes", 2, 11008, 1024, False),
+    ("lanes", 2, 2048, 8192, True),
+    ("lanes", 2, 16384, 8192, True),    # 39.2 / 26.3
+    ("lanes", 3, 4608, 4608, False),    # 8.4 / 12.0
+    ("lanes", 3, 8192, 8192, True),     # 19.1 / 15.1
+    ("lanes", 4, 5632, 4608, False),
+    ("lanes", 4, 5120, 16384, True),    # 28.5 / 20.8
+    ("lanes", 4, 4096, 4096, False),
+    ("lanes", 4, 2304, 6000, True),
+    ("lanes", 8, 2048, 16384, False),   # 8.8 / 9.8
+    ("lanes", 8, 14336, 256, False),    # 9.6 / 11.3
+    ("lanes", 8, 4096, 11008, True),
+    ("lanes", 9, 256, 32000, True),
+    ("lanes", 15, 256, 32000, False),
+    ("native", 3, 5632, 2048, False),
+    ("native", 4, 11008, 4608, False),  # 14.7 / 18.0
+    ("native", 4, 14336, 4608, False),  # 15.7 / 23.4
+    ("native", 4, 11008, 4096, True),
+    ("native", 5, 6144, 64, False),     # 3.9 / 6.9
+    ("native", 8, 4096, 256, False),    # 3.8 / 5.1
+    ("native", 8, 5632, 256, False),    # 4.9 / 6.1
+    ("native", 8, 11008, 4096, True),
+    ("native", 9, 14336, 4608, False),  # 35.3 / 42.4
+    ("native", 12, 4096, 4096, True),
+])
+def test_which_linears_take_the_row_tiles(library, layout: str, rows: int, k: int, n: int, taken: bool) -> None:
+    got = library.linear_takes(int(layout == "lanes"), rows, k // 32, ctypes.c_long(-(-n // 16)), ctypes.c_long(CUS))
+    assert bool(got) is taken
