@@ -518,7 +518,7 @@ bool layout_ok(const Q4Task &t) {
 // 5632 x 2048 40.9 -> 7.2, 64 rows 41.3 -> 14.3, 128 rows 41.2 -> 34.2; 64 rows
 // 2048 x 5632 18.2 -> 12.6, 96 rows 18.1 -> 18.7 (not taken); 24 rows 4096 x 11008
 // 36.8 -> 24.9; 16 rows 2048 x 32000 24.0 -> 16.4, 24 rows 23.8 -> 31.2 (not taken).
-static bool takes_prefill(const Q4Task &t, long tiles) {
+static bool takes_native_prefill(const Q4Task &t, long tiles) {
     const int rpl = fits(t.blocks, 4) ? 4 : 2;
     const double groups = (t.rows + 4 * rpl - 1) / (4 * rpl), chunks = (t.blocks + 31) / 32;
     const double here = 2.5 + 3.6e-3 * (rpl == 4 && t.blocks > 128 ? 1.7 : 1.0) * tiles * groups * chunks;
@@ -529,7 +529,10 @@ static bool takes_prefill(const Q4Task &t, long tiles) {
 int q4_0_rows_linear(const Q4Task &t, hipStream_t stream) {
     if (t.rows < 2 || !layout_ok(t)) return QXT_CAPABILITY_MISSING;
     const long tiles = (t.ncols + 15) / 16, cus = compute_units();
-    if (t.rows > 15 ? !takes_prefill(t, tiles) : !rows_linear_takes(t.lanes != 0, t.rows, t.blocks, tiles, cus)) return QXT_CAPABILITY_MISSING;
+    const bool taken = t.rows < 16 ? rows_linear_takes(t.lanes != 0, t.rows, t.blocks, tiles, cus)
+                       : t.lanes   ? rows_lanes_prefill_takes(t.rows, t.blocks, tiles, cus)
+                                   : takes_native_prefill(t, tiles);
+    if (!taken) return QXT_CAPABILITY_MISSING;
     // The fewest rows per lane that leave every workgroup a CU of its own;
     // larger grids take all rows at once (K = 5632, N = 2048, 5 rows: two row
     // groups 6.4 us, one 7.0; K = 2048, N = 5632: 6.6 and 5.3).

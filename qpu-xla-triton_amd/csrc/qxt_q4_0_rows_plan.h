@@ -219,4 +219,15 @@ inline bool rows_linear_takes(bool lanes, int rows, int blocks, long tiles, long
     return n >= (few ? 192 : 96);
 }
 
+// Sixteen or more rows over lane weights, which the prefill tiles do not read:
+// the other kernels take four rows at a time and read the weights again for each
+// four, these sixteen or eight.  MI355X, us, those -> these: 24 rows 2048 x 32000
+// 52 -> 32, 96 rows 4096 x 4096 53 -> 25, 512 rows 2048 x 5632 181 -> 59; but 16 rows
+// 14336 x 64 9.3 -> 11.2, 64 rows 256 x 11008 7.6 -> 9.9 (few tiles of a long K, many
+// of a K that fills a quarter of a chunk: not taken).
+inline bool rows_lanes_prefill_takes(int rows, int blocks, long tiles, long cus) {
+    const long n = tiles * 256 / cus * ((rows + 15) / 16);
+    return blocks < 16 ? n <= 640 : blocks < 256 || n > 8;
+}
+
 }  // namespace qxt

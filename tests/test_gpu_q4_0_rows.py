@@ -164,6 +164,7 @@ def test_row_tile_batch_captured_and_replayed_reads_the_rows_of_each_replay() ->
                 out.cpu().numpy(), oracle.q4_0_q8_0_reference(oracle.quantize_q8_0_blocks(rows), wt))
 
 
+@pytest.mark.parametrize("layout", ["lanes", "native"])
 @pytest.mark.parametrize("rows,blocks,n,wcol0,ncols", [
     (16, 64, 70, 0, 70),       # a whole group of sixteen rows, or several smaller ones
     (17, 24, 300, 5, 290),     # one row past a group
@@ -174,9 +175,14 @@ def test_row_tile_batch_captured_and_replayed_reads_the_rows_of_each_replay() ->
     (300, 64, 100, 0, 100),
     (64, 64, 5632, 0, 5632),   # the last row count here, the prefill tiles past it
     (96, 64, 5632, 0, 5632),
+    (24, 64, 32000, 0, 32000),  # lanes only from here: more column tiles than a round of them
+    (70, 448, 256, 16, 240),    # a K past two groups' LDS
+    (16, 448, 64, 0, 64),       # the four-row kernels
+    (33, 8, 11008, 0, 11008),
+    (259, 16, 2000, 1, 1990),
 ])
-def test_short_prompts_on_row_tiles_bit_exact(rows: int, blocks: int, n: int, wcol0: int, ncols: int) -> None:
-    _check_linear("native", rows, blocks, n, wcol0, ncols)
+def test_short_prompts_on_row_tiles_bit_exact(layout: str, rows: int, blocks: int, n: int, wcol0: int, ncols: int) -> None:
+    _check_linear(layout, rows, blocks, n, wcol0, ncols)
 
 
 def _check_batch(shapes, source: str, layouts: str, offset: int = 0) -> None:

@@ -31,7 +31,8 @@ extern "C" int plan(const int *chunks, const long *tiles, int n, int cus, double
     return qxt::rows_batch_preferred(t, units, fp32, cus);
 }
 extern "C" int linear_takes(int lanes, int rows, int blocks, long tiles, long cus) {
-    return qxt::rows_linear_takes(lanes, rows, blocks, tiles, cus);
+    return rows < 16 ? qxt::rows_linear_takes(lanes, rows, blocks, tiles, cus)
+                     : qxt::rows_lanes_prefill_takes(rows, blocks, tiles, cus);
 }
 """
 
@@ -162,6 +163,13 @@ def test_which_batches_take_the_row_tiles(library, shapes, fp32: bool, preferred
     ("native", 8, 11008, 4096, True),
     ("native", 9, 14336, 4608, False),  # 35.3 / 42.4
     ("native", 12, 4096, 4096, True),
+    # Lane weights have no prefill tiles to lose to.
+    ("lanes", 16, 2048, 32000, True),
+    ("lanes", 24, 2048, 32000, True),
+    ("lanes", 512, 2048, 5632, True),
+    ("lanes", 16, 14336, 64, False),    # 9.3 / 11.2
+    ("lanes", 64, 256, 11008, False),   # 7.6 / 9.9
+    ("lanes", 64, 14336, 1024, True),
 ])
 def test_which_linears_take_the_row_tiles(library, layout: str, rows: int, k: int, n: int, taken: bool) -> None:
     got = library.linear_takes(int(layout == "lanes"), rows, k // 32, ctypes.c_long(-(-n // 16)), ctypes.c_long(CUS))
