@@ -10,9 +10,10 @@
 // Built with -ffp-contract=off so the two multiplies and the add round
 // separately, which makes the result bit-identical to the NumPy oracle.
 //
-// Tiling (w8a8_gemm_kernel): a 256-thread workgroup (4 waves, 2 x 2) owns a
-// BM x BN output tile; each wave owns a (BM/2) x (BN/2) sub-tile of 32 x 32
-// MFMA blocks.  K advances BKT bytes per stage; A and B tiles live in LDS
+// Tiling (w8a8_gemm_kernel): a group of four waves, 2 x 2, owns a BM x BN
+// output tile, each wave a (BM/2) x (BN/2) sub-tile of 32 x 32 MFMA blocks (one
+// wave along a side of 32); a workgroup holds one group, or up to eight that
+// split K (qxt_w8a8_tiles.h has the choice).  K advances BKT bytes per stage; A and B tiles live in LDS
 // with K contiguous per row, padded by 16 bytes so the 16-byte fragment reads
 // are bank-conflict free.  The large-tile streaming kernel
 // (w8a8_gemm_stream_kernel) uses eight waves of 128 x 64 instead.
@@ -27,6 +28,7 @@
 #include <vector>
 
 #include "qxt_common.h"
+#include "qxt_w8a8_tiles.h"
 
 namespace qxt {
 namespace {
@@ -1256,61 +1258,24 @@ bool gemv_path(int m, int k) {
     return m <= kGemvMaxRows && static_cast<size_t>(rows) * k <= kGemvMaxLds;
 }
 
-// Tiles of problems too small for 256 x 256 ones.  What bounds them is what a CU
-// takes in from L2, measured at 55 to 61 bytes per ns with any of these tiles,
-// so the choice is the largest tile that still gives (nearly) every CU one, with
-// at least two K stages in flight in registers: one stage in flight left each
-// stage waiting for L2 (0.6 us at 64 x 64).  Two groups of four waves per tile
-// (KS = 2) where a CU holds one workgroup.
-// Measured on MI355X, GEMM alone, rotated weights, back to back (M x K x N, us;
-// before: 128 x 128 tiles from one tile per CU, else 64 x 64, one stage in
-// flight):
-//   128 x 128:  512 x 4096 x 14336 55.8 -> 46.5, 1024 x 4096 x 8192 53.2 -> 48.9;
-//               KS = 2: 1024 x 4096 x 4096 44.7 -> 26.9, 256 x 4096 x 14336 36.4 -> 27.2,
-//               256 x 4096 x 11008 (172 tiles) 32.9 -> 26.2; at 141 tiles 23.7
-//               against 21.7 with 64 x 64;
-//   128 x 64:   512 x 14336 x 4096 89.5 -> 51.7 (64 x 64: 62.3), 512 x 4096 x 4096
-//               27.2 -> 18.4; a second round of them (282 tiles) 28.3 against 21.7;
-//   64 x 64:    KS = 2, three stages: 48 x 4096 x 14336 29.1 -> 14.8, 128 x 14336 x
-//               4096 87.4 -> 34.4, 8 x 14336 x 4096 89.0 -> 27.4, 32 x 4096 x 11008
-//               28.3 -> 11.8; past one tile per CU, KS = 1: 300 x 4096 x 6000
-//               29.6 -> 21.7, 64 x 1024 x 32000 13.1 -> 9.7, 768 x 2048 x 5632
-//               24.1 -> 20.2 (128 x 128: 24.4).
-// While even 32 x 32 tiles, or 64 x 32, leave at most one to a CU they take the
-// call from K = 1024: a CU takes in half of the columns or less, and eight or
-// four groups of waves (KS) keep as many loads in flight.  64 x 64 -> 32 x 32:
-// 8 x 14336 x 4096 27.9 -> 21.0, 48 x 14336 x 4096 33.4 -> 22.5, 16 x 14336 x 512
-// 26.7 -> 16.1, 8 x 4096 x 4096 10.4 -> 8.6, packed 8 x 14336 x 4096 48.0 -> 22.2; 512 of
-// K 3.8 -> 4.6, a second round of tiles (8 x 4096 x 8800) 13.0 -> 16.7, not taken.
-// 64 x 64 -> 64 x 32: 128 x 14336 x 4096 35.4 -> 27.8, 200 x 4096 x 2048 10.5 -> 8.9,
-// 40 x 8192 x 8192 24.1 -> 19.2; a second round (64 x 4096 x 11008) 16.4 -> 20.7.
 template <bool K4N>
 int launch_mid(const GemmArgs &args, int epi, uint32_t layout, hipStream_t stream) {
-    const long cus = compute_units();
-    auto tiles = [&](long bm, long bn) { return ((args.m + bm - 1) / bm) * ((args.n + bn - 1) / bn); };
-    const long t128 = tiles(128, 128), t12864 = tiles(128, 64), t64 = tiles(64, 64);
-    if (args.m > 64) {  // fewer rows would leave half of a 128-row tile empty
-        // (Short K over packed weights: their transposing LDS writes make the
-        // longer stage dearer, 2048 x 2048 x 5632 68.1 against 69.8 us.)
-        if (t128 > cus && !(args.k < 3072 && 4 * t128 <= 5 * cus))
-            return K4N && args.k < 3072 ? launch_gemm<128, 128, 64, 1, 1, K4N>(args, epi, layout, stream)
-                                        : launch_gemm<128, 128, 128, 2, 1, K4N>(args, epi, layout, stream);
-        if (t128 <= cus && 8 * t128 >= 5 * cus)
-            return launch_gemm<128, 128, 128, 2, 1, K4N, 2>(args, epi, layout, stream);
-        if (t12864 <= cus && 5 * t12864 >= 4 * cus)
-            return launch_gemm<128, 64, 128, 3, 1, K4N, 2>(args, epi, layout, stream);
+    switch (w8a8_mid_tile(args.m, args.n, args.k, K4N, compute_units())) {
+        case MidTile::k128x128Short: return launch_gemm<128, 128, 64, 1, 1, K4N>(args, epi, layout, stream);
+        case MidTile::k128x128: return launch_gemm<128, 128, 128, 2, 1, K4N>(args, epi, layout, stream);
+        case MidTile::k128x128Groups: return launch_gemm<128, 128, 128, 2, 1, K4N, 2>(args, epi, layout, stream);
+        case MidTile::k128x64Groups: return launch_gemm<128, 64, 128, 3, 1, K4N, 2>(args, epi, layout, stream);
+        case MidTile::k32x32Groups: return launch_gemm<32, 32, 128, 3, 1, K4N, 8>(args, epi, layout, stream);
+        case MidTile::k64x32Groups: return launch_gemm<64, 32, 128, 3, 1, K4N, 4>(args, epi, layout, stream);
+        case MidTile::k64x64Groups: return launch_gemm<64, 64, 128, 3, 1, K4N, 2>(args, epi, layout, stream);
+        default: return launch_gemm<64, 64, 128, 2, 1, K4N>(args, epi, layout, stream);
     }
-    if (args.k >= 1024 && tiles(32, 32) <= cus)
-        return launch_gemm<32, 32, 128, 3, 1, K4N, 8>(args, epi, layout, stream);
-    if (args.k >= 1024 && tiles(64, 32) <= cus)
-        return launch_gemm<64, 32, 128, 3, 1, K4N, 4>(args, epi, layout, stream);
-    if (t64 <= cus) return launch_gemm<64, 64, 128, 3, 1, K4N, 2>(args, epi, layout, stream);
-    return launch_gemm<64, 64, 128, 2, 1, K4N>(args, epi, layout, stream);
 }
 
 int run_gemm(const GemmArgs &args, int epi, uint32_t layout, hipStream_t stream) {
     if (gemv_path(args.m, args.k)) return dispatch_gemv<false>(args, FusedRows{}, epi, layout, stream);
-    // 256 x 256 tiles once they give every CU a workgroup; 128 x 128 below that.
+    // 256 x 256 tiles once they give every CU a workgroup; below that the tiles
+    // of qxt_w8a8_tiles.h.
     const long cus = compute_units();
     const long tm = (args.m + 255) / 256, tn = (args.n + 255) / 256;
     const bool big = tm * tn >= cus;
