@@ -73,9 +73,9 @@ def test_reference_seed_fixture_bit_exact_and_block_dots() -> None:
         (1, 1024, 16),   # K=32768: 128 units per column, two columns per workgroup
         (4, 128, 11000),  # four rows, wide tiles: 43 columns per workgroup in three rounds, ragged last tile
         (8, 128, 4100),   # two row groups of wide tiles, three rounds per workgroup
-        (6, 16, 130),     # four-row matrix-core tiles over native rows, two block ranges per unit
-        (4, 32, 77),      # four block ranges per unit
-        (4, 64, 9000),    # eight block ranges per unit, tiles of several rounds
+        (6, 16, 130),     # 16-row tiles, two units per column
+        (4, 32, 77),      # four
+        (4, 64, 9000),    # four-row matrix-core tiles over native rows, eight units per column, several rounds
         (1, 448, 300),    # K=14336 at one row: split units over 512 threads, 448 Q8_0 blocks fetched
         (1, 512, 200),    # K=16384: the largest row the split single linear fetches into registers
     ],
@@ -493,15 +493,15 @@ def test_lane_pack_kernel_matches_the_layout_definition(n: int, blocks: int) -> 
     (4, 4096, 11000, 8, 10984),  # wide four-row tiles over lane weights, several rounds, ragged
     (1, 5632, 2048, 16, 2032),  # a column range starting inside a lane group
     (2, 256, 37, 5, 31),        # a partial last group, any column range
-    (17, 512, 64, 0, 64),       # rows beyond one MFMA-free row group
+    (17, 512, 64, 0, 64),       # 16-row tiles past one row group
     (4, 14336, 1024, 0, 1024),  # K = 14336 at four rows: one-column tiles above 64 KB of LDS
     (8, 14336, 512, 16, 496),   # two row groups at K = 14336
-    # four-row matrix-core tiles at every block range per unit that divides 16
-    (4, 256, 37, 5, 31),        # one block range per unit, ragged
+    # 16-row tiles at every unit count per column that divides 16
+    (4, 256, 37, 5, 31),        # one unit, ragged
     (6, 512, 130, 2, 128),      # two, a partial second row group
     (5, 1024, 200, 3, 190),     # four, one row in the second row group
     (4, 2048, 300, 0, 300),     # eight
-    (4, 2048, 9000, 3, 8990),   # eight, tiles of several rounds (units over two waves each)
+    (4, 2048, 9000, 3, 8990),   # eight, on four-row tiles of several rounds (units over two waves each)
 ])
 def test_lane_linear_bit_exact_against_oracle(rows: int, k: int, n: int, wcol0: int, ncols: int) -> None:
     rng = np.random.default_rng(5000 + rows + n)

@@ -1,4 +1,5 @@
-"""GPU parity for the Q4_0 kernels over 16-row matrix-core tiles, at the edges of their tiles and rules.
+"""GPU parity for the Q4_0 kernels over 16-row matrix-core tiles, at the edges of their tiles and rules,
+and for what those rules leave to the other kernels.
 
 Every case is compared bit for bit with the oracle: the integer dots are
 exact and the fp32 terms are scaled and added in the oracle's order.
@@ -239,3 +240,45 @@ def test_small_batch_of_mixed_activations_is_one_launch(shapes) -> None:
         _check_batch(shapes, "mixed", "mixed")
     names = [name for name, _ in timing.records if "pack" not in name]
     assert names == ["q4_0_batch_kernel"] * 2
+
+
+@pytest.mark.parametrize("layout,rows,blocks,n,wcol0,ncols", [
+    # Four-row matrix-core tiles at every unit count per column, past the row tiles' column counts.
+    ("lanes", 4, 8, 2104, 4, 2100),
+    ("lanes", 4, 16, 2100, 0, 2100),
+    ("lanes", 4, 32, 2077, 0, 2077),
+    ("lanes", 5, 8, 8300, 0, 8300),      # a second row group of one row
+    ("lanes", 7, 64, 9000, 0, 9000),
+    ("lanes", 6, 128, 6000, 3, 5990),
+    ("native", 4, 8, 8300, 0, 8300),
+    ("native", 4, 16, 8305, 5, 8300),
+    ("native", 4, 32, 8300, 0, 8300),
+    ("native", 6, 128, 4200, 0, 4200),
+    # v_dot4 tiles over lanes, and blocks over lanes of a wave: a second round of row tiles, few columns of a long K.
+    ("lanes", 2, 176, 4200, 0, 4200),
+    ("lanes", 3, 144, 4200, 1, 4190),
+    ("lanes", 4, 176, 4300, 0, 4300),
+    ("lanes", 12, 344, 200, 0, 200),
+    ("native", 8, 176, 256, 0, 256),
+    ("native", 10, 448, 4608, 0, 4608),
+])
+def test_linears_left_to_the_other_kernels_bit_exact(layout: str, rows: int, blocks: int, n: int, wcol0: int,
+                                                     ncols: int) -> None:
+    _check_linear(layout, rows, blocks, n, wcol0, ncols)
+
+
+@pytest.mark.parametrize("layouts", ["lanes", "native", "mixed"])
+@pytest.mark.parametrize("source", ["fp32", "native", "mixed"])
+@pytest.mark.parametrize("shapes", [
+    [(4, 8, 17000), (2, 8, 17000), (3, 8, 500)],    # chunks mostly empty, in kernel arguments
+    [(4, 8, 9000)] * 4 + [(2, 16, 500), (3, 8, 33)],  # and in device tables
+    [(4, 776, 40), (2, 64, 300)],                   # K past the row tiles' LDS
+    [(2, 776, 33), (3, 8, 100), (4, 64, 70), (1, 16, 5), (4, 784, 16)],
+])
+def test_multi_row_batches_left_to_the_v_dot4_kernel_bit_exact(shapes, source: str, layouts: str) -> None:
+    _check_batch(shapes, source, layouts)
+
+
+@pytest.mark.parametrize("shapes", [[(4, 64, 700), (1, 8, 16), (3, 176, 130)], [(2, 40, 200)] * 5])
+def test_multi_row_batch_of_activations_two_bytes_off_a_word_bit_exact(shapes) -> None:
+    _check_batch(shapes, "native", "mixed", offset=2)

@@ -124,6 +124,8 @@ def test_small_grids_of_a_longer_k_take_it_in_one_pass(library) -> None:
     ([(256, 32000)] * 8 + [(2048, 2048)] * 8, False, False),   # chunks mostly empty
     ([(256, 32000)] * 8 + [(2048, 2048)] * 8, True, False),
     ([(256, 512), (512, 512)], False, True),                    # the same, few tiles
+    ([(256, 17000), (256, 17000), (256, 500)], True, False),
+    ([(256, 9000)] * 4 + [(512, 500), (256, 33)], False, False),
     ([(1024, 4096), (24576, 128)], False, False),               # passes over a very long K, little else
     ([(1024, 4096), (24576, 128)], True, True),                 # quantised here
     ([(1024, 32000), (24576, 2048)], False, True),
@@ -163,6 +165,22 @@ def test_which_batches_take_the_row_tiles(library, shapes, fp32: bool, preferred
     ("native", 8, 11008, 4096, True),
     ("native", 9, 14336, 4608, False),  # 35.3 / 42.4
     ("native", 12, 4096, 4096, True),
+    # The linears that the GPU tests hold for the other kernels.
+    ("lanes", 4, 256, 2100, False),
+    ("lanes", 4, 512, 2100, False),
+    ("lanes", 4, 1024, 2077, False),
+    ("lanes", 5, 256, 8300, False),
+    ("lanes", 7, 2048, 9000, False),
+    ("lanes", 6, 4096, 5990, False),
+    ("native", 4, 256, 8300, False),
+    ("native", 4, 512, 8300, False),
+    ("native", 4, 1024, 8300, False),
+    ("native", 6, 4096, 4200, False),
+    ("lanes", 2, 5632, 4200, False),
+    ("lanes", 3, 4608, 4190, False),
+    ("lanes", 4, 5632, 4300, False),
+    ("lanes", 12, 11008, 200, False),
+    ("native", 10, 14336, 4608, False),
     # Lane weights have no prefill tiles to lose to.
     ("lanes", 16, 2048, 32000, True),
     ("lanes", 24, 2048, 32000, True),
